@@ -508,7 +508,7 @@ int build_query_matrix(jhq_index* ix) {
     JHQ_HIP(hipMemcpyAsync(ix->dqmat.p, ix->dP.p, static_cast<size_t>(d) * d * sizeof(float),
                            hipMemcpyDeviceToDevice, ix->stream));
     JHQ_HIP(jhq::gemm_nt_store(ix->dcent.p, d, dpt.p, d, nlist, d, d,
-                               ix->dqmat.p + static_cast<size_t>(d) * d, d, false, ix->stream));
+                               ix->dqmat.p + static_cast<size_t>(d) * d, d, ix->stream));
     JHQ_HIP(hipStreamSynchronize(ix->stream));
     return JHQ_OK;
 }
@@ -1296,7 +1296,7 @@ int train_impl(jhq_index* ix, const float* x, int64_t n_train) {
     JHQ_TRY(dx.upload(x, static_cast<size_t>(n_train) * d));
     JHQ_TRY(dy.alloc(static_cast<size_t>(n_train) * d));
     JHQ_TRY(dcodes.alloc(static_cast<size_t>(n_train) * M));
-    JHQ_HIP(jhq::gemm_nt_store(dx.p, d, ix->dP.p, d, n_train, d, d, dy.p, d, false, ix->stream));
+    JHQ_HIP(jhq::gemm_nt_store(dx.p, d, ix->dP.p, d, n_train, d, d, dy.p, d, ix->stream));
     JHQ_HIP(jhq::encode(dy.p, n_train, d, M, Ds, ix->K1D, ix->bpd, ix->dc1d.p, ix->Kr, 1, ix->Br,
                         ix->bpv, nullptr, dcodes.p, nullptr, nullptr, 1, ix->stream));
     dx.release();
@@ -1551,7 +1551,7 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
             JHQ_HIP(hipStreamWaitEvent(s, sy.copied[i], 0));
             if (dtype != JHQ_F32)
                 JHQ_HIP(jhq::convert_to_f32(draw[i].p, dtype, static_cast<int64_t>(cnt), dxb[i].p, s));
-            JHQ_HIP(jhq::gemm_nt_store(dxb[i].p, d, ix->dP.p, d, nb, d, d, dyb.p, d, false, s));
+            JHQ_HIP(jhq::gemm_nt_store(dxb[i].p, d, ix->dP.p, d, nb, d, d, dyb.p, d, s));
             JHQ_HIP(hipEventRecord(sy.consumed[i], s));
             JHQ_HIP(jhq::encode(dyb.p, nb, d, M, ix->Ds, ix->K1D, ix->bpd, ix->dc1d.p, ix->Kr, ix->RC,
                                 ix->Br, bpv, ix->dres_c1d.p, dpc.p + start * M,
@@ -2153,7 +2153,7 @@ int jhq_get_timing(const jhq_index* idx, double* ms, int n_ms, int64_t* batches)
 
 int jhq_k_rotate(const float* d_P, const float* d_x, int64_t n, int d, float* d_y, void* stream) {
     if (!d_P || !d_x || !d_y || n < 0 || d <= 0) return fail(JHQ_EINVAL, "bad argument");
-    JHQ_HIP(jhq::gemm_nt_store(d_x, d, d_P, d, n, d, d, d_y, d, n < 1024,
+    JHQ_HIP(jhq::gemm_nt_store(d_x, d, d_P, d, n, d, d, d_y, d,
                                static_cast<hipStream_t>(stream)));
     return JHQ_OK;
 }

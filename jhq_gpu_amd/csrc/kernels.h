@@ -11,21 +11,17 @@ constexpr int kLdsBytes = 160 * 1024;
 // Candidates per padded group of the per-list code-major layout.
 constexpr int kGroup = 16;
 
-// C[i][j] = sum_k A[i][k] * Bm[j][k] as an fmaf chain, k ascending from 0.
+// C[i][j] = sum_k A[i][k] * Bm[j][k] as an fmaf chain, k ascending from 0
+// (on fp32 MFMA, gemm_chain.hip).
 //   store : C[i*ldc + j] = acc
-//   score : C[i*ldc + j] = fmaf(-2, acc, norms[j])     (= norms[j] - 2 acc)
 //   argmin: keys[i] = min over j of (ord(fmaf(-2, acc, norms[j])) << 32 | j)
 //           (keys must be pre-filled with ~0)
 hipError_t gemm_nt_store(const float* A, int64_t lda, const float* Bm, int64_t ldb,
-                         int64_t n, int m, int d, float* C, int64_t ldc,
-                         bool small_rows, hipStream_t s);
-hipError_t gemm_nt_score(const float* A, int64_t lda, const float* Bm, int64_t ldb,
-                         int64_t n, int m, int d, const float* norms, float* C,
-                         int64_t ldc, bool small_rows, hipStream_t s);
+                         int64_t n, int m, int d, float* C, int64_t ldc, hipStream_t s);
 hipError_t gemm_nt_argmin(const float* A, int64_t lda, const float* Bm, int64_t ldb,
                           int64_t n, int m, int d, const float* norms,
                           unsigned long long* keys, hipStream_t s);
-// EPI argmin over the rows rowidx[0 .. min(n_max, *ndev)) of A (ndev read on
+// The argmin over the rows rowidx[0 .. min(n_max, *ndev)) of A (ndev read on
 // the device); keys[i] belongs to row rowidx[i].
 hipError_t gemm_nt_argmin_rows(const float* A, int64_t lda, const int32_t* rowidx,
                                const int32_t* ndev, int64_t n_max, const float* Bm, int64_t ldb,

@@ -295,277 +295,14 @@ __device__ __forceinline__ int block_topk(GetV getv, GetT gett, int n, int k, in
 }
 
 // ---------------------------------------------------------------------------
-// Fixed-order SIMT GEMM  C = A * Bm^T  (both operands k-contiguous rows)
+// Fixed-order argmin over listed rows
 // ---------------------------------------------------------------------------
-enum { EPI_STORE = 0, EPI_SCORE = 1, EPI_ARGMIN = 2 };
+enum { EPI_STORE = 0, EPI_SCORE = 1 };
 
-template <int BM, int BN, int BK, int TM, int TN, int EPI>
-__global__ void __launch_bounds__((BM / TM) * (BN / TN))
-gemm_nt_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ Bm,
-               int64_t ldb, int64_t n, int m, int d, float* __restrict__ C, int64_t ldc,
-               const float* __restrict__ norms, unsigned long long* __restrict__ amin) {
-    constexpr int TX = BN / TN, TY = BM / TM, NT = TX * TY;
-    constexpr int AL = BM * BK / NT, BL = BN * BK / NT;
-    static_assert((BM * BK) % NT == 0 && (BN * BK) % NT == 0, "tile/threads mismatch");
-    static_assert(TX <= 64 && (TX & (TX - 1)) == 0, "TX must be a power of two <= 64");
-    __shared__ __align__(16) float As[2][BK][BM + 4];
-    __shared__ __align__(16) float Bs[2][BK][BN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid % TX, ty = tid / TX;
-    const int64_t row0 = (int64_t)blockIdx.y * BM;
-    const int col0 = blockIdx.x * BN;
-
-    float ra[AL], rb[BL];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < AL; i++) {
-            const int e = tid + i * NT, r = e / BK, kk = e % BK;
-            const int64_t gr = row0 + r;
-            const int gk = k0 + kk;
-            ra[i] = (gr < n && gk < d) ? A[gr * lda + gk] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < BL; i++) {
-            const int e = tid + i * NT, r = e / BK, kk = e % BK;
-            const int gc = col0 + r, gk = k0 + kk;
-            rb[i] = (gc < m && gk < d) ? Bm[(int64_t)gc * ldb + gk] : 0.0f;
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < AL; i++) {
-            const int e = tid + i * NT;
-            As[buf][e % BK][e / BK] = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < BL; i++) {
-            const int e = tid + i * NT;
-            Bs[buf][e % BK][e / BK] = rb[i];
-        }
-    };
-    // thread's rows / cols: groups of 4 interleaved across the tile when
-    // TM (TN) is a multiple of 4, contiguous otherwise.
-    auto row_of = [&](int i) {
-        return (TM % 4 == 0) ? (i / 4) * (TY * 4) + ty * 4 + (i % 4) : ty * TM + i;
-    };
-    auto col_of = [&](int j) {
-        return (TN % 4 == 0) ? (j / 4) * (TX * 4) + tx * 4 + (j % 4) : tx * TN + j;
-    };
-
-    float acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = 0.0f;
-
-    const int nk = (d + BK - 1) / BK;
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int t = 0; t < nk; t++) {
-        const int buf = t & 1;
-        if (t + 1 < nk) gload((t + 1) * BK);
-#pragma unroll
-        for (int kk = 0; kk < BK; kk++) {
-            float a[TM], b[TN];
-#pragma unroll
-            for (int i = 0; i < TM; i++) a[i] = As[buf][kk][row_of(i)];
-#pragma unroll
-            for (int j = 0; j < TN; j++) b[j] = Bs[buf][kk][col_of(j)];
-#pragma unroll
-            for (int i = 0; i < TM; i++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        if (t + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-
-    if constexpr (EPI == EPI_ARGMIN) {
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int64_t gr = row0 + row_of(i);
-            unsigned long long best = ~0ull;
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int gc = col0 + col_of(j);
-                if (gc < m) {
-                    const float sc = fmaf(-2.0f, acc[i][j], norms[gc]);
-                    const unsigned long long key =
-                        ((unsigned long long)f2ord(sc) << 32) | (unsigned long long)(uint32_t)gc;
-                    best = key < best ? key : best;
-                }
-            }
-#pragma unroll
-            for (int off = TX / 2; off > 0; off >>= 1) {
-                const unsigned long long o = __shfl_xor(best, off);
-                best = o < best ? o : best;
-            }
-            if (tx == 0 && gr < n && best != ~0ull) atomicMin(&amin[gr], best);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < TM; i++) {
-            const int64_t gr = row0 + row_of(i);
-            if (gr >= n) continue;
-#pragma unroll
-            for (int j = 0; j < TN; j++) {
-                const int gc = col0 + col_of(j);
-                if (gc >= m) continue;
-                float v = acc[i][j];
-                if constexpr (EPI == EPI_SCORE) v = fmaf(-2.0f, v, norms[gc]);
-                C[gr * ldc + gc] = v;
-            }
-        }
-    }
-}
-
-template <int BM, int BN, int BK, int TM, int TN, int EPI>
-static hipError_t launch_gemm(const float* A, int64_t lda, const float* Bm, int64_t ldb,
-                              int64_t n, int m, int d, float* C, int64_t ldc, const float* norms,
-                              unsigned long long* amin, hipStream_t s) {
-    constexpr int NT = (BM / TM) * (BN / TN);
-    if (n <= 0 || m <= 0) return hipSuccess;
-    // rows go on grid.y; launch in chunks of at most 65535 row tiles.
-    const int64_t rows_per_launch = (int64_t)BM * 65535;
-    for (int64_t r0 = 0; r0 < n; r0 += rows_per_launch) {
-        const int64_t nr = (n - r0) < rows_per_launch ? (n - r0) : rows_per_launch;
-        dim3 grid((m + BN - 1) / BN, (unsigned)((nr + BM - 1) / BM));
-        hipLaunchKernelGGL((gemm_nt_kernel<BM, BN, BK, TM, TN, EPI>), grid, dim3(NT), 0, s,
-                           A + r0 * lda, lda, Bm, ldb, nr, m, d,
-                           C ? C + r0 * ldc : nullptr, ldc, norms, amin ? amin + r0 : nullptr);
-    }
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Skinny fixed-order GEMM for a query batch: C[b][j] = sum_k A[b][k] Bm[j][k]
-// with nb <= a few hundred rows and many columns.  One output column per
-// lane, TQ batch rows per wave, 4 waves per workgroup sharing one 64-column
-// B tile staged k-major in LDS; A values are LDS broadcasts.  The k loop is
-// ascending, so every output is the same fmaf chain as the SIMT tile kernel.
-// ---------------------------------------------------------------------------
-#ifndef JHQ_SKINNY_BK
-#define JHQ_SKINNY_BK 128
-#endif
-template <int TQ, int EPI>
-__global__ void __launch_bounds__(256)
-gemm_skinny_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ Bm,
-                   int64_t ldb, int nb, int m, int d, float* __restrict__ C, int64_t ldc,
-                   const float* __restrict__ norms) {
-    constexpr int BK = JHQ_SKINNY_BK, QW = 4 * TQ;
-    constexpr int BL = 64 * BK / 256;             // B floats per thread per tile
-    constexpr int QL = (QW * BK + 255) / 256;     // A floats per thread per tile
-    __shared__ float Bs[2][BK][65];
-    __shared__ __align__(16) float Qs[2][BK][QW];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int j0 = blockIdx.x * 64, b0 = blockIdx.y * QW;
-    float rb[BL], rq[QL];
-    auto gload = [&](int k0) {
-#pragma unroll
-        for (int i = 0; i < BL; i++) {
-            const int e = tid + i * 256, r = e / BK, kk = e % BK;
-            const int gj = j0 + r, gk = k0 + kk;
-            rb[i] = (gj < m && gk < d) ? Bm[(int64_t)gj * ldb + gk] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < QL; i++) {
-            const int e = tid + i * 256, r = e / BK, kk = e % BK;
-            const int gb = b0 + r, gk = k0 + kk;
-            rq[i] = (e < QW * BK && gb < nb && gk < d) ? A[(int64_t)gb * lda + gk] : 0.0f;
-        }
-    };
-    auto sstore = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < BL; i++) {
-            const int e = tid + i * 256;
-            Bs[buf][e % BK][e / BK] = rb[i];
-        }
-#pragma unroll
-        for (int i = 0; i < QL; i++) {
-            const int e = tid + i * 256;
-            if (e < QW * BK) Qs[buf][e % BK][e / BK] = rq[i];
-        }
-    };
-    float acc[TQ];
-#pragma unroll
-    for (int t = 0; t < TQ; t++) acc[t] = 0.0f;
-    const int nk = (d + BK - 1) / BK;
-    gload(0);
-    sstore(0);
-    __syncthreads();
-    for (int t = 0; t < nk; t++) {
-        const int buf = t & 1;
-        if (t + 1 < nk) gload((t + 1) * BK);
-#pragma unroll 16
-        for (int kk = 0; kk < BK; kk++) {
-            const float bv = Bs[buf][kk][lane];
-#pragma unroll
-            for (int u = 0; u < TQ; u++) acc[u] = fmaf(Qs[buf][kk][w * TQ + u], bv, acc[u]);
-        }
-        if (t + 1 < nk) sstore(buf ^ 1);
-        __syncthreads();
-    }
-    const int j = j0 + lane;
-    if (j < m) {
-#pragma unroll
-        for (int u = 0; u < TQ; u++) {
-            const int b = b0 + w * TQ + u;
-            if (b < nb) {
-                float v = acc[u];
-                if constexpr (EPI == EPI_SCORE) v = fmaf(-2.0f, v, norms[j]);
-                C[(int64_t)b * ldc + j] = v;
-            }
-        }
-    }
-}
-
-template <int EPI>
-static hipError_t launch_skinny(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb,
-                                int m, int d, float* C, int64_t ldc, const float* norms,
-                                hipStream_t s) {
-    // about 2048 waves: TQ = rows per wave, a power of two in [1, 8]
-    const int64_t colblocks = (m + 63) / 64;
-    int TQ = 1;
-    while (TQ < 8 && colblocks * ((nb + TQ - 1) / TQ) > 2048) TQ *= 2;
-    dim3 grid((unsigned)colblocks, (unsigned)((nb + 4 * TQ - 1) / (4 * TQ)));
-    switch (TQ) {
-        case 1: hipLaunchKernelGGL((gemm_skinny_kernel<1, EPI>), grid, dim3(256), 0, s, A, lda, Bm, ldb, nb, m, d, C, ldc, norms); break;
-        case 2: hipLaunchKernelGGL((gemm_skinny_kernel<2, EPI>), grid, dim3(256), 0, s, A, lda, Bm, ldb, nb, m, d, C, ldc, norms); break;
-        case 4: hipLaunchKernelGGL((gemm_skinny_kernel<4, EPI>), grid, dim3(256), 0, s, A, lda, Bm, ldb, nb, m, d, C, ldc, norms); break;
-        default: hipLaunchKernelGGL((gemm_skinny_kernel<8, EPI>), grid, dim3(256), 0, s, A, lda, Bm, ldb, nb, m, d, C, ldc, norms); break;
-    }
-    return hipGetLastError();
-}
-
-hipError_t gemm_nt_store(const float* A, int64_t lda, const float* Bm, int64_t ldb, int64_t n,
-                         int m, int d, float* C, int64_t ldc, bool small_rows, hipStream_t s) {
-    if (small_rows && n <= 4096)
-        return launch_skinny<EPI_STORE>(A, lda, Bm, ldb, (int)n, m, d, C, ldc, nullptr, s);
-    return launch_gemm<128, 128, 16, 8, 8, EPI_STORE>(A, lda, Bm, ldb, n, m, d, C, ldc, nullptr,
-                                                       nullptr, s);
-}
-
-hipError_t gemm_nt_score(const float* A, int64_t lda, const float* Bm, int64_t ldb, int64_t n,
-                         int m, int d, const float* norms, float* C, int64_t ldc,
-                         bool small_rows, hipStream_t s) {
-    if (small_rows && n <= 4096)
-        return launch_skinny<EPI_SCORE>(A, lda, Bm, ldb, (int)n, m, d, C, ldc, norms, s);
-    return launch_gemm<128, 128, 16, 8, 8, EPI_SCORE>(A, lda, Bm, ldb, n, m, d, C, ldc, norms,
-                                                       nullptr, s);
-}
-
-hipError_t gemm_nt_argmin(const float* A, int64_t lda, const float* Bm, int64_t ldb, int64_t n,
-                          int m, int d, const float* norms, unsigned long long* keys,
-                          hipStream_t s) {
-    return launch_gemm<128, 128, 16, 8, 8, EPI_ARGMIN>(A, lda, Bm, ldb, n, m, d, nullptr, 0,
-                                                        norms, keys, s);
-}
-
-// EPI_ARGMIN over listed rows: keys[i] = the smallest
+// keys[i] = the smallest
 // (f2ord(fmaf(-2, dot, norms[c])) << 32 | c) over the lists c, for the row
 // A[rowidx[i]], i < min(n_max, *ndev); each dot the fmaf chain in k order,
-// as in gemm_nt_kernel.  The listed rows are few (the near ties of an
+// as in gemm_chain_kernel.  The listed rows are few (the near ties of an
 // assignment): a workgroup takes 128 lists, one per thread, and steps over
 // groups of 8 rows staged in LDS; each list value read feeds the group's 8
 // chains, and each row's minimum goes out as one atomic per wave.
