@@ -45,21 +45,32 @@ __device__ __forceinline__ uint32_t chain_ord(float f) {
 // operands, which leaves the chain's value.  Workgroups go to the 8 XCDs in
 // turn; the column tiles of a row tile take consecutive slots of one XCD, so
 // its rows come from that XCD's L2 after the first.
-template <int T, int EPI, bool VEC>
+// With ROWS, row i of A is A[rowidx[i]], i < min(n, *ndev) (the count read on the
+// device), and the workgroups step over the tiles.
+template <int T, int EPI, bool VEC, bool ROWS = false>
 __global__ void __launch_bounds__(256, 2)
 gemm_chain_kernel(const float* __restrict__ A, int64_t lda, const float* __restrict__ Bm,
                   int64_t ldb, int64_t n, int m, int d, float* __restrict__ C, int64_t ldc,
-                  const float* __restrict__ norms, unsigned long long* __restrict__ keys) {
+                  const float* __restrict__ norms, unsigned long long* __restrict__ keys,
+                  const int32_t* __restrict__ rowidx = nullptr,
+                  const int32_t* __restrict__ ndev = nullptr) {
     constexpr int BT = 64 * T, L = BT * kChainBK / 4 / 256;  // float4 per thread and operand
     __shared__ __align__(16) float As[BT][kChainLd];
     __shared__ __align__(16) float Bs[BT][kChainLd];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int l32 = lane & 31, h = lane >> 5, wr = wv >> 1, wc = wv & 1;
     const int ncol = (m + BT - 1) / BT;
-    const int xcd = (int)(blockIdx.x & 7), slot = (int)(blockIdx.x >> 3);
-    const int64_t row0 = (xcd + 8 * (int64_t)(slot / ncol)) * BT;
-    const int col0 = slot % ncol * BT;
-    if (row0 >= n) return;
+    if (ROWS) n = min(n, (int64_t)*ndev);
+    // (without ROWS the grid covers the tiles: one pass)
+    for (int64_t item = blockIdx.x;; item += gridDim.x) {
+    const int64_t slot = item >> 3;
+    const int64_t row0 = ((item & 7) + 8 * (slot / ncol)) * BT;
+    const int col0 = (int)(slot % ncol) * BT;
+    if (row0 >= n) {
+        if (!ROWS || slot / ncol * 8 * BT >= n) return;
+        continue;
+    }
+    if (ROWS) __syncthreads();  // the previous tile's reads are done
 
     // thread t stages 4 k from 4 (t % 8) of rows t / 8 + 32 i
     const int lk = 4 * (tid & 7), lr = tid >> 3;
@@ -67,7 +78,8 @@ gemm_chain_kernel(const float* __restrict__ A, int64_t lda, const float* __restr
     const float* bp[L];
 #pragma unroll
     for (int i = 0; i < L; i++) {
-        ap[i] = A + min(row0 + lr + 32 * i, n - 1) * lda;
+        const int64_t row = min(row0 + lr + 32 * i, n - 1);
+        ap[i] = A + (ROWS ? (int64_t)rowidx[row] : row) * lda;
         bp[i] = Bm + (int64_t)min(col0 + lr + 32 * i, m - 1) * ldb;
     }
     float4 ra[L], rb[L];
@@ -213,6 +225,8 @@ gemm_chain_kernel(const float* __restrict__ A, int64_t lda, const float* __restr
             if (!(l32 & 1) && row < n && key != ~0ull) atomicMin(&keys[row], key);
         }
     }
+    if (!ROWS) return;
+    }
 }
 
 template <int T, int EPI>
@@ -231,7 +245,8 @@ static hipError_t launch_chain(const float* A, int64_t lda, const float* Bm, int
         const dim3 grid((unsigned)((rt + 7) / 8 * 8 * ncol));
         auto* k = vec ? gemm_chain_kernel<T, EPI, true> : gemm_chain_kernel<T, EPI, false>;
         hipLaunchKernelGGL(k, grid, dim3(256), 0, s, A + r0 * lda, lda, Bm, ldb, nr, m, d,
-                           C ? C + r0 * ldc : nullptr, ldc, norms, keys ? keys + r0 : nullptr);
+                           C ? C + r0 * ldc : nullptr, ldc, norms, keys ? keys + r0 : nullptr,
+                           (const int32_t*)nullptr, (const int32_t*)nullptr);
     }
     return hipGetLastError();
 }
@@ -260,6 +275,23 @@ hipError_t gemm_nt_argmin(const float* A, int64_t lda, const float* Bm, int64_t 
     return chain_small(n, m)
                ? launch_chain<1, CHAIN_ARGMIN>(A, lda, Bm, ldb, n, m, d, nullptr, 0, norms, keys, s)
                : launch_chain<2, CHAIN_ARGMIN>(A, lda, Bm, ldb, n, m, d, nullptr, 0, norms, keys, s);
+}
+
+// The grid fills the chip for any count; with no row listed it ends at once.
+hipError_t gemm_nt_argmin_rows(const float* A, int64_t lda, const int32_t* rowidx,
+                               const int32_t* ndev, int64_t n_max, const float* Bm, int64_t ldb,
+                               int m, int d, const float* norms, unsigned long long* keys,
+                               hipStream_t s) {
+    if (n_max <= 0 || m <= 0) return hipSuccess;
+    const bool vec = d % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && ((uintptr_t)A & 15) == 0 &&
+                     ((uintptr_t)Bm & 15) == 0;
+    auto* k = vec ? gemm_chain_kernel<1, CHAIN_ARGMIN, true, true>
+                  : gemm_chain_kernel<1, CHAIN_ARGMIN, false, true>;
+    const int64_t tiles = (n_max + 63) / 64 * ((m + 63) / 64);
+    hipLaunchKernelGGL(k, dim3((unsigned)std::min<int64_t>((tiles + 7) / 8 * 8, 1024)), dim3(256), 0,
+                       s, A, lda, Bm, ldb, n_max, m, d, (float*)nullptr, (int64_t)0, norms, keys,
+                       rowidx, ndev);
+    return hipGetLastError();
 }
 
 }  // namespace jhq

@@ -466,7 +466,7 @@ int assign_rows(jhq_index* ix, const float* d_y, int64_t n, int32_t* d_assign,
         JHQ_HIP(jhq::assign_mfma(d_y, n, ix->d, ix->dcent.p, ix->nlist, ix->dnorms.p, d_assign,
                                  ix->dascr.p, ix->dascr.n, keys.p, ix->stream));
         if (verbose() && ix->drecheck.p)
-            JHQ_HIP(jhq::assign_mfma_tally(ix->dascr.p, n, ix->drecheck.p, ix->stream));
+            JHQ_HIP(jhq::assign_mfma_tally(ix->dascr.p, ix->drecheck.p, ix->stream));
         return JHQ_OK;
     }
     JHQ_HIP(jhq::fill_u64(keys.p, n, ~0ull, ix->stream));
@@ -2186,18 +2186,17 @@ int jhq_k_assign(const float* d_y, int64_t n, int d, const float* d_cent, const 
     if (!d_y || !d_cent || !d_cent_norms || !d_assign || n < 0 || d <= 0 || nlist <= 0)
         return fail(JHQ_EINVAL, "bad argument");
     hipStream_t s = static_cast<hipStream_t>(stream);
+    // keys, then the MFMA pass's scratch (16-byte aligned)
+    const bool mfma = jhq::assign_mfma_ok(d, d_y, d_cent) && (n + 127) / 128 <= 65535;
+    const size_t nk = static_cast<size_t>((std::max<int64_t>(n, 1) + 31) / 32 * 32);
+    const size_t sf = mfma ? jhq::assign_mfma_scratch_floats(std::max<int64_t>(n, 1), d, nlist) : 0;
     unsigned long long* keys = nullptr;
-    JHQ_HIP(hipMallocAsync(reinterpret_cast<void**>(&keys), std::max<int64_t>(n, 1) * 8, s));
+    JHQ_HIP(hipMallocAsync(reinterpret_cast<void**>(&keys), nk * 8 + sf * sizeof(float), s));
     hipError_t e = hipSuccess;
-    if (jhq::assign_mfma_ok(d, d_y, d_cent) && (n + 127) / 128 <= 65535) {
+    if (mfma) {
         // MFMA scores, fixed-order re-check of near ties: the same lists
-        const size_t sf = jhq::assign_mfma_scratch_floats(std::max<int64_t>(n, 1), d, nlist);
-        float* scr = nullptr;
-        e = hipMallocAsync(reinterpret_cast<void**>(&scr), sf * sizeof(float), s);
-        if (e == hipSuccess) {
-            e = jhq::assign_mfma(d_y, n, d, d_cent, nlist, d_cent_norms, d_assign, scr, sf, keys, s);
-            (void)hipFreeAsync(scr, s);
-        }
+        e = jhq::assign_mfma(d_y, n, d, d_cent, nlist, d_cent_norms, d_assign,
+                             reinterpret_cast<float*>(keys + nk), sf, keys, s);
     } else {
         e = jhq::fill_u64(keys, n, ~0ull, s);
         if (e == hipSuccess) e = jhq::gemm_nt_argmin(d_y, d, d_cent, d, n, nlist, d, d_cent_norms, keys, s);

@@ -29,8 +29,9 @@ hipError_t gemm_nt_argmin_rows(const float* A, int64_t lda, const int32_t* rowid
                                hipStream_t s);
 // IVF assignment on bf16 MFMA (each float split into two bf16, three
 // products per pair) with the fixed-order argmin re-checking every row whose
-// two best approximate scores are closer than the error bound
-// (assign_mfma.hip); the result equals gemm_nt_argmin's bit for bit.
+// two best approximate scores are closer than the error bound over the lists
+// that the bound leaves (assign_mfma.hip); the result equals gemm_nt_argmin's
+// bit for bit.
 // scratch: assign_mfma_scratch_floats(n, d, nlist) floats; keys: n u64.
 // Enqueue only.
 bool assign_mfma_ok(int d, const float* Y, const float* Cm);
@@ -38,12 +39,9 @@ size_t assign_mfma_scratch_floats(int64_t n, int d, int nlist);
 hipError_t assign_mfma(const float* Y, int64_t n, int d, const float* Cm, int nlist,
                        const float* norms, int32_t* assign, float* scratch,
                        size_t scratch_floats, unsigned long long* keys, hipStream_t s);
-// The number of rows the last assign_mfma on this scratch re-checked
-// (device int).
-const int32_t* assign_mfma_rechecked(const float* scratch, int64_t n);
-// *total += that count (on the stream)
-hipError_t assign_mfma_tally(const float* scratch, int64_t n, unsigned long long* total,
-                             hipStream_t s);
+// *total += the number of rows the last assign_mfma on this scratch re-checked
+// (on the stream)
+hipError_t assign_mfma_tally(const float* scratch, unsigned long long* total, hipStream_t s);
 // The same products on fp32 MFMA for the query side (rotation, centroid
 // scores); not a fixed summation order, so only distances and near-tie probe
 // choices depend on it, never the stored codes.

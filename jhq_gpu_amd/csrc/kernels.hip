@@ -295,132 +295,6 @@ __device__ __forceinline__ int block_topk(GetV getv, GetT gett, int n, int k, in
 }
 
 // ---------------------------------------------------------------------------
-// Fixed-order argmin over listed rows
-// ---------------------------------------------------------------------------
-enum { EPI_STORE = 0, EPI_SCORE = 1 };
-
-// keys[i] = the smallest
-// (f2ord(fmaf(-2, dot, norms[c])) << 32 | c) over the lists c, for the row
-// A[rowidx[i]], i < min(n_max, *ndev); each dot the fmaf chain in k order,
-// as in gemm_chain_kernel.  The listed rows are few (the near ties of an
-// assignment): a workgroup takes 128 lists, one per thread, and steps over
-// groups of 8 rows staged in LDS; each list value read feeds the group's 8
-// chains, and each row's minimum goes out as one atomic per wave.
-constexpr int kArgRows = 8, kArgCols = 128, kArgK = 512, kArgKB = 64;
-
-__global__ void __launch_bounds__(kArgCols)
-argmin_rows_kernel(const float* __restrict__ A, int64_t lda, const int32_t* __restrict__ rowidx,
-                   const int32_t* __restrict__ ndev, int64_t n_max, const float* __restrict__ Bm,
-                   int64_t ldb, int m, int d, const float* __restrict__ norms,
-                   unsigned long long* __restrict__ keys) {
-    __shared__ __align__(16) float ys[kArgRows][kArgK];
-    const int tid = threadIdx.x;
-    const int col = blockIdx.x * kArgCols + tid;
-    int64_t cnt = *ndev;
-    if (cnt > n_max) cnt = n_max;
-    const float* brow = Bm + (int64_t)(col < m ? col : 0) * ldb;
-    const bool vec = (ldb % 4) == 0 && ((uintptr_t)Bm & 15) == 0;
-    for (int64_t g0 = (int64_t)blockIdx.y * kArgRows; g0 < cnt;
-         g0 += (int64_t)gridDim.y * kArgRows) {
-        const int nr = (cnt - g0) < kArgRows ? (int)(cnt - g0) : kArgRows;
-        int64_t rbase[kArgRows];
-#pragma unroll
-        for (int i = 0; i < kArgRows; i++) rbase[i] = (int64_t)rowidx[g0 + (i < nr ? i : nr - 1)] * lda;
-        float acc[kArgRows];
-#pragma unroll
-        for (int i = 0; i < kArgRows; i++) acc[i] = 0.0f;
-        for (int k0 = 0; k0 < d; k0 += kArgK) {
-            const int kw = (d - k0) < kArgK ? (d - k0) : kArgK;
-            // all of the chunk's loads in flight at once (rows past nr and
-            // k past kw read a valid element and store zero)
-            constexpr int kPer = kArgRows * kArgK / kArgCols;
-            static_assert(kArgK % kArgCols == 0, "a thread's elements stay in one row per k block");
-            float v[kPer];
-#pragma unroll
-            for (int t = 0; t < kPer; t++) {
-                const int e = tid + t * kArgCols, i = e / kArgK, kk = e % kArgK;
-                const int kc = kk < kw ? kk : kw - 1;
-                v[t] = A[rbase[i] + k0 + kc];
-            }
-            __syncthreads();  // the previous chunk's reads are done
-#pragma unroll
-            for (int t = 0; t < kPer; t++) {
-                const int e = tid + t * kArgCols, i = e / kArgK, kk = e % kArgK;
-                ys[i][kk] = (i < nr && kk < kw) ? v[t] : 0.0f;
-            }
-            __syncthreads();
-            if (col < m) {
-                int kk = 0;
-                if (vec && kw >= kArgKB) {
-                    // the list's values kArgKB at a time, the next kArgKB
-                    // loading while these feed the chains
-                    constexpr int J = kArgKB / 4;
-                    const int kend = kw / kArgKB * kArgKB;
-                    float4 cur[J], nxt[J];
-#pragma unroll
-                    for (int j = 0; j < J; j++) cur[j] = *(const float4*)(brow + k0 + 4 * j);
-                    for (; kk < kend; kk += kArgKB) {
-                        if (kk + kArgKB < kend) {
-#pragma unroll
-                            for (int j = 0; j < J; j++)
-                                nxt[j] = *(const float4*)(brow + k0 + kk + kArgKB + 4 * j);
-                        }
-#pragma unroll
-                        for (int j = 0; j < J; j++) {
-                            const float4 b = cur[j];
-#pragma unroll
-                            for (int i = 0; i < kArgRows; i++) {
-                                const float4 a = *(const float4*)&ys[i][kk + 4 * j];
-                                acc[i] = fmaf(a.x, b.x, acc[i]);
-                                acc[i] = fmaf(a.y, b.y, acc[i]);
-                                acc[i] = fmaf(a.z, b.z, acc[i]);
-                                acc[i] = fmaf(a.w, b.w, acc[i]);
-                            }
-                        }
-#pragma unroll
-                        for (int j = 0; j < J; j++) cur[j] = nxt[j];
-                    }
-                }
-                for (; kk < kw; kk++) {
-                    const float b = brow[k0 + kk];
-#pragma unroll
-                    for (int i = 0; i < kArgRows; i++) acc[i] = fmaf(ys[i][kk], b, acc[i]);
-                }
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kArgRows; i++) {
-            if (i >= nr) break;
-            unsigned long long key = ~0ull;
-            if (col < m) {
-                const float sc = fmaf(-2.0f, acc[i], norms[col]);
-                key = ((unsigned long long)f2ord(sc) << 32) | (unsigned long long)(uint32_t)col;
-            }
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                const unsigned long long o = __shfl_xor(key, off);
-                key = o < key ? o : key;
-            }
-            if ((tid & 63) == 0 && key != ~0ull) atomicMin(&keys[g0 + i], key);
-        }
-    }
-}
-
-hipError_t gemm_nt_argmin_rows(const float* A, int64_t lda, const int32_t* rowidx,
-                               const int32_t* ndev, int64_t n_max, const float* Bm, int64_t ldb,
-                               int m, int d, const float* norms, unsigned long long* keys,
-                               hipStream_t s) {
-    if (n_max <= 0 || m <= 0) return hipSuccess;
-    // up to 32 workgroup rows step over the groups of rows below the count
-    // read on the device
-    const int64_t groups = (n_max + kArgRows - 1) / kArgRows;
-    dim3 grid((m + kArgCols - 1) / kArgCols, (unsigned)(groups < 32 ? groups : 32));
-    hipLaunchKernelGGL(argmin_rows_kernel, grid, dim3(kArgCols), 0, s, A, lda, rowidx, ndev, n_max,
-                       Bm, ldb, m, d, norms, keys);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // Query-side GEMMs on fp32 MFMA (v_mfma_f32_16x16x4f32):
 //   C[b][n] = sum_k A[b][k] * Bm[n][k]      (EPI_STORE: query rotation)
 //   C[b][n] = norms[n] - 2 * that           (EPI_SCORE: centroid scores)
@@ -433,6 +307,8 @@ hipError_t gemm_nt_argmin_rows(const float* A, int64_t lda, const int32_t* rowid
 // workgroup split K and their partial tiles are added in LDS in wave order.
 // ---------------------------------------------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));
+
+enum { EPI_STORE = 0, EPI_SCORE = 1 };
 
 template <int S, int EPI, bool VEC>
 __global__ void __launch_bounds__(64 * S)
