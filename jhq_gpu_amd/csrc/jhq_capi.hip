@@ -586,6 +586,7 @@ int ensure_workspace(jhq_index* ix, Workspace& w, int ck, int k, int P, int max_
 bool skew_eligible(const jhq_index* ix) { return ix->M % 32 == 0 && ix->M <= 128; }
 
 bool rows_wanted(const jhq_index* ix);
+size_t rows_need(const jhq_index* ix, int64_t cap);
 
 // The pre-scan computes 16-query tiles over every probed list; it pays off
 // when the queries of a batch share their lists so that the tiles are mostly
@@ -742,8 +743,7 @@ int refresh_skew(jhq_index* ix) {
 int refresh_rows(jhq_index* ix) {
     if (!ix->rows_stale) return JHQ_OK;
     const int nl = ix->nlist;
-    const size_t need = static_cast<size_t>((std::max<int64_t>(ix->pool_cap, 1) + 15) / 16 * 16) *
-                        static_cast<size_t>(ix->M);
+    const size_t need = rows_need(ix, ix->pool_cap);
     if (ix->dcodes_r.n < need || static_cast<int>(ix->rows_start.size()) != nl) {
         // (the old copy may still be read by enqueued work)
         if (ix->dcodes_r.n < need) {
@@ -1409,6 +1409,28 @@ int grow_pool(jhq_index* ix, int64_t need) {
     return JHQ_OK;
 }
 
+// Bytes of the row-major copy for a pool of `cap` slots.
+size_t rows_need(const jhq_index* ix, int64_t cap) {
+    return static_cast<size_t>((std::max<int64_t>(cap, 1) + 15) / 16 * 16) *
+           static_cast<size_t>(ix->M);
+}
+
+// Whether the row-major copy is kept and covers the pool, so that inserts write
+// it as they go (refresh_rows writes what they did not).
+bool rows_live(const jhq_index* ix) {
+    return rows_wanted(ix) && ix->dcodes_r.n >= rows_need(ix, ix->pool_cap) &&
+           static_cast<int>(ix->rows_start.size()) == ix->nlist;
+}
+
+// The lists move to `nstart` and their rows with them: those the copy holds
+// whole are current there, the others are written by the next refresh.
+void move_rows(jhq_index* ix, const std::vector<int32_t>& nstart) {
+    for (int l = 0; l < ix->nlist; l++) {
+        const bool whole = ix->rows_start[l] == ix->l_start[l] && ix->rows_rows[l] == ix->l_size[l];
+        ix->rows_start[l] = whole ? nstart[l] : -1;
+    }
+}
+
 // Re-packs every list into a new pool: list l gets capacity
 // round16(need[l] * 5/4) (need = its size after the pending insert), blocks
 // are laid out in list order, dead blocks left by earlier moves are dropped,
@@ -1438,14 +1460,24 @@ int repack_pool(jhq_index* ix, const std::vector<int64_t>& need) {
     JHQ_TRY(nr.alloc(static_cast<size_t>(pcap) * bpv));
     JHQ_TRY(nco.alloc(static_cast<size_t>(pcap)));
     JHQ_TRY(ni.alloc(static_cast<size_t>(pcap)));
+    // the row-major copy moves along where it is kept (without memory for its
+    // new buffer the next refresh writes it)
+    DBuf<uint8_t> nrow;
+    const bool rows = rows_live(ix) && nrow.alloc(rows_need(ix, pcap)) == JHQ_OK;
     hipStream_t s = ix->stream;
     if (!moves.empty()) {
         DBuf<int4> dmoves;
         JHQ_TRY(dmoves.upload(moves.data(), moves.size()));
         JHQ_HIP(jhq::relocate_lists(dmoves.p, static_cast<int>(moves.size() / 2), M, bpv,
                                     ix->dcodes_t.p, nc.p, ix->dres.p, nr.p, ix->dcorr.p, nco.p,
-                                    ix->dlist_ids.p, ni.p, s));
+                                    ix->dlist_ids.p, ni.p, rows ? ix->dcodes_r.p : nullptr,
+                                    rows ? nrow.p : nullptr, s));
         JHQ_HIP(hipStreamSynchronize(s));
+    }
+    if (rows) {
+        std::swap(ix->dcodes_r.p, nrow.p);
+        std::swap(ix->dcodes_r.n, nrow.n);
+        move_rows(ix, nstart);
     }
     std::swap(ix->dcodes_t.p, nc.p);
     std::swap(ix->dcodes_t.n, nc.n);
@@ -1638,8 +1670,9 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
             JHQ_HIP(jhq::relocate_lists(dmoves.p, static_cast<int>(moves.size() / 2), M, bpv,
                                         ix->dcodes_t.p, ix->dcodes_t.p, ix->dres.p, ix->dres.p,
                                         ix->dcorr.p, ix->dcorr.p, ix->dlist_ids.p, ix->dlist_ids.p,
-                                        s));
-            JHQ_HIP(hipStreamSynchronize(s));
+                                        rows_live(ix) ? ix->dcodes_r.p : nullptr,
+                                        rows_live(ix) ? ix->dcodes_r.p : nullptr, s));
+            if (rows_live(ix)) move_rows(ix, nstart);
         }
         ix->l_start = nstart;
         ix->l_cap = ncap;
@@ -1656,10 +1689,26 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
         JHQ_TRY(dslist.ensure(static_cast<size_t>(n)));
         JHQ_TRY(dsidx.ensure(static_cast<size_t>(n)));
         JHQ_HIP(jhq::scatter_plan(sorted, first, ix->dldesc.p, n, dorder.p, dslist.p, dsidx.p, s));
+        // the new rows go to the row-major copy as well; a first insert sets it up
+        if (rows_wanted(ix) && ix->ntotal == 0 &&
+            ix->dcodes_r.ensure(rows_need(ix, ix->pool_cap)) == JHQ_OK) {
+            ix->rows_start = ix->l_start;
+            ix->rows_rows.assign(nlist, 0);
+        }
+        const bool rows = rows_live(ix);
         JHQ_HIP(jhq::scatter_lists(dorder.p, dslist.p, dsidx.p, n, id_base, ix->dldesc.p, dpc.p,
                                    drc.p, dco.p, M, bpv, ix->dlist_ids.p, ix->dcodes_t.p, ix->dres.p,
-                                   ix->dcorr.p, s));
-        for (int l = 0; l < nlist; l++) ix->l_size[l] += static_cast<int32_t>(add[l + 1]);
+                                   ix->dcorr.p, rows ? ix->dcodes_r.p : nullptr, s));
+        for (int l = 0; l < nlist; l++) {
+            const int32_t grown = static_cast<int32_t>(add[l + 1]);
+            if (rows && ix->l_size[l] == 0) {
+                ix->rows_start[l] = ix->l_start[l];
+                ix->rows_rows[l] = 0;
+            }
+            if (rows && ix->rows_start[l] == ix->l_start[l] && ix->rows_rows[l] == ix->l_size[l])
+                ix->rows_rows[l] += grown;
+            ix->l_size[l] += grown;
+        }
     }
     // the descriptors with the new sizes follow the scatter on s; the host
     // does not wait (device searches wait for the tail event)

@@ -116,7 +116,9 @@ hipError_t scatter_plan(const unsigned long long* sorted, const int64_t* first, 
 // are indexed by slot.
 //
 // Scatter: new vector s goes to list slist[s] at index sidx[s]; its id is
-// id_base + order[s], order[s] indexing the per-vector inputs pc/rc/co.
+// id_base + order[s], order[s] indexing the per-vector inputs pc/rc/co.  rows
+// (may be null; M a multiple of 4): the row-major copy of the primary codes
+// takes the new rows too.
 // Lane-skewed rows of the primary codes (row[t] = code[(t - i mod 32) mod M]
 // for candidate i of each list, the wrapped bytes t < i mod 32 stored as
 // code + 1 mod 256), in blocks of 16 slots stored piece by piece (16 bytes of
@@ -126,6 +128,11 @@ hipError_t scatter_plan(const unsigned long long* sorted, const int64_t* first, 
 hipError_t skew_codes(const int4* ldesc, const int32_t* from, int nlist, int max_rows,
                       const uint8_t* codes_t, int M, uint8_t* skew, hipStream_t s);
 int64_t skew_bytes(int64_t pool_cap, int M);
+// Byte offset of the 16-byte piece q of slot p's skewed row (blocks of 16 slots).
+__host__ __device__ inline int64_t skew_piece(int64_t p, int q, int M) {
+    return ((p >> 4) * (M >> 4) + q) * 256 + (p & 15) * 16;
+}
+
 // Row-major copy of the primary codes (slot p's M bytes at rows[p * M],
 // pool_cap * M bytes; M a multiple of 16), rows from[l] .. size-1 of each
 // list l (from rounded down to 16).
@@ -134,13 +141,17 @@ hipError_t row_codes(const int4* ldesc, const int32_t* from, int nlist, int max_
 hipError_t scatter_lists(const int32_t* order, const int32_t* slist, const int32_t* sidx,
                          int64_t n, int64_t id_base, const int4* ldesc, const uint8_t* pc,
                          const uint8_t* rc, const float* co, int M, int bpv, int32_t* ids_out,
-                         uint8_t* codes_t, uint8_t* res_out, float* corr_out, hipStream_t s);
+                         uint8_t* codes_t, uint8_t* res_out, float* corr_out, uint8_t* rows,
+                         hipStream_t s);
 // Moves list blocks: moves[2r] = {start, cap, size} (source), moves[2r+1] =
-// {start, cap} (destination); blocks must not overlap.
+// {start, cap} (destination); blocks must not overlap, and the padding after
+// a block's size candidates up to the next multiple of 16 may be written.
+// rows_dst (may be null): the row-major copy moves along.
 hipError_t relocate_lists(const int4* moves, int nmoves, int M, int bpv, const uint8_t* codes_src,
                           uint8_t* codes_dst, const uint8_t* res_src, uint8_t* res_dst,
                           const float* corr_src, float* corr_dst, const int32_t* ids_src,
-                          int32_t* ids_dst, hipStream_t s);
+                          int32_t* ids_dst, const uint8_t* rows_src, uint8_t* rows_dst,
+                          hipStream_t s);
 
 // The integer-MFMA pre-scan's share of the probe selection (see mfma_scan):
 // its workspace (ws, ws_bytes, laid out for Bcap queries) and dump buffer

@@ -778,330 +778,6 @@ hipError_t keys_to_assign(const unsigned long long* keys, int64_t n, int32_t* as
 }
 
 // ---------------------------------------------------------------------------
-// Encode: a workgroup takes kEncV vectors and walks their dimensions in
-// chunks of kEncC.  Every thread quantizes dimensions of the chunk (reads of
-// consecutive floats of one vector), the digits and residual indices are
-// packed into code and residual bytes from LDS, and one lane per vector
-// carries that vector's residual correction: a sequential fmaf chain in
-// dimension order over the quantized values the chunk left in LDS.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int nearest_mid(const float* mids, int n, float v) {
-    int lo = 0, hi = n - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (v < mids[mid]) hi = mid;
-        else lo = mid + 1;
-    }
-    return lo;
-}
-
-constexpr int kEncV = 16, kEncC = 128, kEncT = 256;
-constexpr int kEncPer = kEncV * kEncC / kEncT;  // dimensions a thread quantizes per chunk
-
-__global__ void __launch_bounds__(kEncT)
-encode_kernel(const float* __restrict__ y, int64_t n, int d, int M, int Ds, int K1D, int bpd,
-              const float* __restrict__ c1d, int Kr, int RC, int Br, int bpv,
-              const float* __restrict__ res_c1d, uint8_t* __restrict__ codes,
-              uint8_t* __restrict__ res, float* __restrict__ corr, int mode) {
-    // RC residual codebooks of Kr words: one shared by every dimension (the
-    // reference, v14/jhq_gpu_index.cu:302-330) or one per subspace (RC = M)
-    __shared__ float cval[256], cmid[256];
-    // the chunk's quantized values (yhat, rhat) per vector; the odd row
-    // stride puts the chain lanes' reads of one column in distinct banks
-    __shared__ float yh[kEncV][kEncC + 1], rh[kEncV][kEncC + 1];
-    __shared__ uint8_t dg[kEncV][kEncC], rq[kEncV][kEncC];
-    extern __shared__ float rsh[];  // rval[RC*Kr], rmid[RC*Kr]
-    float* rval = rsh;
-    float* rmid = rsh + RC * Kr;
-    const int tid = threadIdx.x;
-    const int64_t v0 = (int64_t)blockIdx.x * kEncV;
-    const int nv = (n - v0) < kEncV ? (int)(n - v0) : kEncV;
-    if (tid < K1D) cval[tid] = c1d[tid];
-    if (mode & 2)
-        for (int i = tid; i < RC * Kr; i += kEncT) rval[i] = res_c1d[i];
-    __syncthreads();
-    if (tid + 1 < K1D) cmid[tid] = 0.5f * (cval[tid] + cval[tid + 1]);
-    if (mode & 2)
-        for (int i = tid; i < RC * Kr; i += kEncT)
-            if ((i % Kr) + 1 < Kr) rmid[i] = 0.5f * (rval[i] + rval[i + 1]);
-    __syncthreads();
-    const int kmask = K1D - 1;
-    float dot = 0.0f;  // lane v < nv: vector v0 + v's chain
-    for (int c0 = 0; c0 < d; c0 += kEncC) {
-        const int cw = (d - c0) < kEncC ? (d - c0) : kEncC;
-        float val[kEncPer];
-#pragma unroll
-        for (int i = 0; i < kEncPer; i++) {
-            const int e = tid + i * kEncT, v = e / kEncC, jj = e % kEncC;
-            val[i] = (v < nv && jj < cw) ? y[(v0 + v) * d + c0 + jj] : 0.0f;
-        }
-#pragma unroll
-        for (int i = 0; i < kEncPer; i++) {
-            const int e = tid + i * kEncT, v = e / kEncC, jj = e % kEncC;
-            if (v >= nv || jj >= cw) continue;
-            const int j = c0 + jj;
-            const int m = j / Ds, k = j - m * Ds;
-            int dig;
-            if (mode & 1) dig = (K1D == 1) ? 0 : nearest_mid(cmid, K1D, val[i]);
-            else dig = (codes[(v0 + v) * M + m] >> (k * bpd)) & kmask;
-            dg[v][jj] = (uint8_t)dig;
-            if (mode & 2) {
-                const int cb = (RC == 1) ? 0 : m;
-                const float yhat = cval[dig];
-                const float r = val[i] - yhat;
-                const int ri = (Kr == 1) ? 0 : nearest_mid(rmid + cb * Kr, Kr, r);
-                rq[v][jj] = (uint8_t)ri;
-                yh[v][jj] = yhat;
-                rh[v][jj] = rval[cb * Kr + ri];
-            }
-        }
-        __syncthreads();
-        if (mode & 1) {
-            // whole subspaces of the chunk (c0 is a multiple of Ds, which divides 32)
-            const int ms = cw / Ds;
-            for (int e = tid; e < kEncV * ms; e += kEncT) {
-                const int v = e / ms, mm = e - v * ms;
-                if (v >= nv) continue;
-                uint32_t code = 0u;
-                for (int k = 0; k < Ds; k++) code |= (uint32_t)dg[v][mm * Ds + k] << (k * bpd);
-                codes[(v0 + v) * M + c0 / Ds + mm] = (uint8_t)code;
-            }
-        }
-        if (mode & 2) {
-            if (Br == 4) {
-                // two dimensions a byte, the even one in the low nibble; an odd
-                // last dimension alone in the low nibble of the last byte
-                const int nb = (cw + 1) >> 1;
-                for (int e = tid; e < kEncV * nb; e += kEncT) {
-                    const int v = e / nb, b = e - v * nb;
-                    if (v >= nv) continue;
-                    const uint32_t lo = rq[v][2 * b] & 0x0Fu;
-                    const uint32_t hi = (2 * b + 1 < cw) ? (rq[v][2 * b + 1] & 0x0Fu) : 0u;
-                    res[(v0 + v) * bpv + (c0 >> 1) + b] = (uint8_t)(lo | (hi << 4));
-                }
-            } else {
-                for (int e = tid; e < kEncV * cw; e += kEncT) {
-                    const int v = e / cw, jj = e - v * cw;
-                    if (v >= nv) continue;
-                    res[(v0 + v) * bpv + c0 + jj] = rq[v][jj];
-                }
-            }
-            if (tid < nv)
-                for (int jj = 0; jj < cw; jj++) dot = fmaf(yh[tid][jj], rh[tid][jj], dot);
-        }
-        __syncthreads();
-    }
-    if ((mode & 2) && tid < nv) corr[v0 + tid] = 2.0f * dot;
-}
-
-hipError_t encode(const float* y, int64_t n, int d, int M, int Ds, int K1D, int bpd,
-                  const float* c1d, int Kr, int RC, int Br, int bpv, const float* res_c1d,
-                  uint8_t* codes, uint8_t* res, float* corr, int mode, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    if (K1D > 256 || Kr > 256 || (32 % Ds) != 0 || (RC != 1 && RC != M) || Ds * M != d ||
-        ((mode & 2) && Br != 4 && Br != 8))
-        return hipErrorInvalidValue;
-    const size_t lds = (size_t)2 * RC * Kr * sizeof(float);
-    if (lds > 96 * 1024) return hipErrorInvalidValue;
-    if (lds > 48 * 1024) {
-        static const hipError_t e = hipFuncSetAttribute((const void*)encode_kernel,
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                         96 * 1024);
-        if (e != hipSuccess) return e;
-    }
-    const int64_t blocks = (n + kEncV - 1) / kEncV;
-    if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(encode_kernel, dim3((unsigned)blocks), dim3(kEncT), lds, s, y, n, d, M, Ds,
-                       K1D, bpd, c1d, Kr, RC, Br, bpv, res_c1d, codes, res, corr, mode);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// List storage.  The lists live in one pool of padded candidate slots; list l
-// is described by ListDesc {start, cap, size, cbase} (int4): it owns slots
-// [start, start + cap) (cap a multiple of 16) and holds size candidates.
-// Primary codes are code-major inside the block: byte m of candidate i is at
-// codes_t[start*M + m*cap + i], so one 32-bit load returns byte m of four
-// consecutive candidates.  Residual codes, corrections and ids are indexed by
-// slot.  cbase is the list's first canonical position (lists in list order,
-// candidates in insertion order), the tag the exact selection breaks ties
-// with, so results do not depend on where a list's block sits in the pool.
-// ---------------------------------------------------------------------------
-__global__ void scatter_kernel(const int32_t* __restrict__ order, const int32_t* __restrict__ slist,
-                               const int32_t* __restrict__ sidx, int64_t n, int64_t id_base,
-                               const int4* __restrict__ ldesc, const uint8_t* __restrict__ pc,
-                               const uint8_t* __restrict__ rc, const float* __restrict__ co, int M,
-                               int bpv, int32_t* __restrict__ ids_out, uint8_t* __restrict__ codes_t,
-                               uint8_t* __restrict__ res_out, float* __restrict__ corr_out) {
-    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int64_t id = order[s];
-    const int4 L = ldesc[slist[s]];
-    const int64_t i = sidx[s];
-    const int64_t slot = (int64_t)L.x + i;
-    ids_out[slot] = (int32_t)(id + id_base);
-    corr_out[slot] = co[id];
-    uint8_t* dst = codes_t + (int64_t)L.x * M + i;
-    const uint8_t* src = pc + id * M;
-    for (int m = 0; m < M; m++) dst[(int64_t)m * L.y] = src[m];
-    const uint8_t* rs = rc + id * bpv;
-    uint8_t* rd = res_out + slot * bpv;
-    for (int b2 = 0; b2 < bpv; b2++) rd[b2] = rs[b2];
-}
-
-// ---------------------------------------------------------------------------
-// Lane-skewed copy of the primary codes, for the scan that runs each lane a
-// fixed number of subspaces behind its neighbours.  Candidate i of a list
-// (pool slot p = start + i) gets M bytes
-//   row[t] = code[t - s]                 for t >= s = i mod 32,
-//   row[t] = (code[M + t - s] + 1) mod 256 for t < s,
-// so that at step t the lane holding i reads subspace t - s from row
-// position t.  The tail bytes (t < s, read one period later, with the next
-// candidate's head bytes) are raised by one LUT row: their LUT address
-// (v + 1) * M + t - s is then the head bytes' formula, and code 255 wraps to
-// the copy of row 255's last subspaces kept just below the LUT.
-// The rows are stored in blocks of 16 slots (list starts and capacities are
-// multiples of 16), piece by piece: the 16 bytes row[16q .. 16q+15] of slot p
-// are at skew_piece(p, q) = ((p / 16) * (M / 16) + q) * 256 + (p mod 16) * 16,
-// so the 64 lanes of a wave reading one piece of their candidates (four
-// blocks of 16 consecutive slots) touch four 256-byte runs.
-// Rows from[l] .. size-1 of list l are written (with the rest of the first
-// block, whose rows are current anyway); one thread per piece, the codes read
-// from the code-major blocks (codes_t[start * M + m * cap + i]).
-// ---------------------------------------------------------------------------
-__host__ __device__ inline int64_t skew_piece(int64_t p, int q, int M) {
-    return ((p >> 4) * (M >> 4) + q) * 256 + (p & 15) * 16;
-}
-
-__global__ void skew_codes_kernel(const int4* __restrict__ ldesc, const int32_t* __restrict__ from,
-                                  const uint8_t* __restrict__ codes_t, int M,
-                                  uint8_t* __restrict__ skew) {
-    const int4 L = ldesc[blockIdx.x];
-    const int q = threadIdx.x >> 4;
-    if (q >= M / 16) return;
-    // blocks of 16 slots; grid-y strides over the list's blocks
-    for (int64_t i = (int64_t)(from[blockIdx.x] & ~15) + (int64_t)blockIdx.y * 16 + (threadIdx.x & 15);
-         i < L.z; i += (int64_t)gridDim.y * 16) {
-        const uint8_t* src = codes_t + (int64_t)L.x * M + i;
-        const int s = (int)(i & 31);
-        uint32_t w[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            w[k] = 0u;
-#pragma unroll
-            for (int e = 0; e < 4; e++) {
-                int m = 16 * q + 4 * k + e - s;
-                // tail bytes (t < s) hold code + 1 (mod 256)
-                const uint32_t inc = m < 0 ? 1u : 0u;
-                if (m < 0) m += M;
-                w[k] |= ((src[(int64_t)m * L.y] + inc) & 0xffu) << (8 * e);
-            }
-        }
-        *(uint4*)(skew + skew_piece((int64_t)L.x + i, q, M)) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-}
-
-int64_t skew_bytes(int64_t pool_cap, int M) { return (pool_cap + 15) / 16 * 16 * M; }
-
-// Row-major copy of the primary codes: slot p's M bytes at rows[p * M], so
-// that one vector's codes are one contiguous run (the pre-scan's re-check
-// reads whole rows of a few candidates).  Rows from[l] .. size-1 of list l
-// (from rounded down to 16); thread (16-byte piece q, slot i % 16).
-__global__ void row_codes_kernel(const int4* __restrict__ ldesc, const int32_t* __restrict__ from,
-                                 const uint8_t* __restrict__ codes_t, int M,
-                                 uint8_t* __restrict__ rows) {
-    const int4 L = ldesc[blockIdx.x];
-    const int q = threadIdx.x >> 4;
-    if (q >= M / 16) return;
-    for (int64_t i = (int64_t)(from[blockIdx.x] & ~15) + (int64_t)blockIdx.y * 16 + (threadIdx.x & 15);
-         i < L.z; i += (int64_t)gridDim.y * 16) {
-        const uint8_t* src = codes_t + (int64_t)L.x * M + i;
-        uint32_t w[4];
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            w[k] = 0u;
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                w[k] |= (uint32_t)src[(int64_t)(16 * q + 4 * k + e) * L.y] << (8 * e);
-        }
-        *(uint4*)(rows + ((int64_t)L.x + i) * M + 16 * q) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-}
-
-hipError_t row_codes(const int4* ldesc, const int32_t* from, int nlist, int max_rows,
-                     const uint8_t* codes_t, int M, uint8_t* rows, hipStream_t s) {
-    if (nlist <= 0 || max_rows <= 0) return hipSuccess;
-    const int64_t gy = std::min<int64_t>(((int64_t)max_rows + 15 + 15) / 16, 65535);
-    if (M % 16 != 0 || M > 256) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(row_codes_kernel, dim3(nlist, (unsigned)gy), dim3(M), 0, s, ldesc, from,
-                       codes_t, M, rows);
-    return hipGetLastError();
-}
-
-hipError_t skew_codes(const int4* ldesc, const int32_t* from, int nlist, int max_rows,
-                      const uint8_t* codes_t, int M, uint8_t* skew, hipStream_t s) {
-    if (nlist <= 0 || max_rows <= 0) return hipSuccess;
-    // one block of threads per 16 slots; from[l] is rounded down to 16
-    // (a list of any length: the kernel strides over grid-y)
-    const int64_t gy = std::min<int64_t>(((int64_t)max_rows + 15 + 15) / 16, 65535);
-    if (M % 32 != 0 || M > 256) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(skew_codes_kernel, dim3(nlist, (unsigned)gy), dim3(M), 0, s, ldesc, from,
-                       codes_t, M, skew);
-    return hipGetLastError();
-}
-
-hipError_t scatter_lists(const int32_t* order, const int32_t* slist, const int32_t* sidx,
-                         int64_t n, int64_t id_base, const int4* ldesc, const uint8_t* pc,
-                         const uint8_t* rc, const float* co, int M, int bpv, int32_t* ids_out,
-                         uint8_t* codes_t, uint8_t* res_out, float* corr_out, hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    const int64_t blocks = (n + 255) / 256;
-    hipLaunchKernelGGL(scatter_kernel, dim3((unsigned)blocks), dim3(256), 0, s, order, slist, sidx,
-                       n, id_base, ldesc, pc, rc, co, M, bpv, ids_out, codes_t, res_out, corr_out);
-    return hipGetLastError();
-}
-
-// Moves list blocks.  moves[2r] = {start, cap, size} of block r's source,
-// moves[2r+1] = {start, cap} of its destination; the size candidates are
-// copied and the code-major primary codes re-strided.  Source and
-// destination blocks never overlap (destinations lie past every live block,
-// or in another pool).
-__global__ void relocate_kernel(const int4* __restrict__ moves, int M, int bpv,
-                                const uint8_t* __restrict__ codes_src, uint8_t* __restrict__ codes_dst,
-                                const uint8_t* __restrict__ res_src, uint8_t* __restrict__ res_dst,
-                                const float* __restrict__ corr_src, float* __restrict__ corr_dst,
-                                const int32_t* __restrict__ ids_src, int32_t* __restrict__ ids_dst) {
-    const int4 fr = moves[blockIdx.x * 2];
-    const int4 to = moves[blockIdx.x * 2 + 1];
-    const int size = fr.z;
-    if (size <= 0) return;
-    const uint8_t* cs = codes_src + (int64_t)fr.x * M;
-    uint8_t* cd = codes_dst + (int64_t)to.x * M;
-    for (int64_t e = threadIdx.x; e < (int64_t)M * size; e += blockDim.x) {
-        const int64_t m = e / size, i = e - m * size;
-        cd[m * to.y + i] = cs[m * fr.y + i];
-    }
-    const uint8_t* rs = res_src + (int64_t)fr.x * bpv;
-    uint8_t* rd = res_dst + (int64_t)to.x * bpv;
-    for (int64_t e = threadIdx.x; e < (int64_t)size * bpv; e += blockDim.x) rd[e] = rs[e];
-    for (int i = threadIdx.x; i < size; i += blockDim.x) {
-        corr_dst[to.x + i] = corr_src[fr.x + i];
-        ids_dst[to.x + i] = ids_src[fr.x + i];
-    }
-}
-
-hipError_t relocate_lists(const int4* moves, int nmoves, int M, int bpv, const uint8_t* codes_src,
-                          uint8_t* codes_dst, const uint8_t* res_src, uint8_t* res_dst,
-                          const float* corr_src, float* corr_dst, const int32_t* ids_src,
-                          int32_t* ids_dst, hipStream_t s) {
-    if (nmoves <= 0) return hipSuccess;
-    hipLaunchKernelGGL(relocate_kernel, dim3((unsigned)nmoves), dim3(256), 0, s, moves, M, bpv,
-                       codes_src, codes_dst, res_src, res_dst, corr_src, corr_dst, ids_src,
-                       ids_dst);
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
 // Streaming exact top-k.
 //
 // The candidates of one selection arrive in rounds: in each round every
