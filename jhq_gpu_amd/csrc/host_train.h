@@ -5,7 +5,11 @@
 // file is compiled with -ffp-contract=off and uses fmaf() exactly where the
 // reference's -O3 -march=native build contracts a multiply-add.
 #pragma once
+#include <algorithm>
 #include <cstdint>
+#include <exception>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace jhq {
@@ -24,7 +28,40 @@ std::vector<float> lloyd_max_c1d(float sigma, int K1D);
 float estimate_sigma(const float* x, int64_t n, int d);
 
 // cpu/codebook.cpp:8-58 — 1-D Lloyd k-means with quantile initialisation.
-std::vector<float> train_1d_kmeans(const float* vals, int64_t n, int Kr, int max_iter = 25);
+std::vector<float> train_1d_kmeans(const float* vals, int64_t n, int Kr, int max_iter = 25,
+                                   unsigned max_threads = 16);
+
+// Threads a training step may use.
+inline unsigned host_threads() {
+    return std::max(1u, std::min(std::thread::hardware_concurrency(), 16u));
+}
+
+// Runs f(t) for t < T on T threads (the caller's among them; the caller's alone
+// takes over what no thread could be started for).  An exception of f reaches
+// the caller once every thread has ended.
+template <class F>
+void parallel(unsigned T, F f) {
+    std::vector<std::exception_ptr> err(T);
+    auto call = [&](unsigned t) {
+        try {
+            f(t);
+        } catch (...) {
+            err[t] = std::current_exception();
+        }
+    };
+    std::vector<std::thread> th;
+    th.reserve(T);
+    unsigned started = 1;
+    try {
+        for (; started < T; started++) th.emplace_back(call, started);
+    } catch (const std::system_error&) {
+    }
+    call(0);
+    for (unsigned t = started; t < T; t++) call(t);
+    for (auto& t : th) t.join();
+    for (auto& e : err)
+        if (e) std::rethrow_exception(e);
+}
 
 // cpu/jl_transform.cpp:25-56 — Gaussian fill in column-major storage order,
 // Householder QR (LAPACK xGEQR2/xORG2R conventions, computed in double).

@@ -350,7 +350,9 @@ struct jhq_index {
         for (int l = 0; ok && l < kLanes; l++) ok = hipEventCreate(&e1[l]) == hipSuccess;
         // the span from the first lane's start to the last lane's end
         auto span = [&](const int* ls, int m, float* ms) {
-            constexpr int kIters = 200000;  // a few hundred us
+            // about 270 us (200000 steps took 2.7 ms, and the 20 or so runs of a new
+            // index's calibration 28 of its add()'s 31 ms)
+            constexpr int kIters = 20000;
             if (hipEventRecord(e0, lane[ls[0]]) != hipSuccess) return false;
             for (int i = 1; i < m; i++)
                 if (hipStreamWaitEvent(lane[ls[i]], e0, 0) != hipSuccess) return false;
@@ -1324,19 +1326,31 @@ int train_impl(jhq_index* ix, const float* x, int64_t n_train) {
         std::fprintf(stderr, "[jhq] train: %d residual codebook(s) over %lld values each\n", ix->RC,
                      static_cast<long long>(n_train) * (ix->RC == 1 ? d : Ds));
     ix->res_c1d.assign(static_cast<size_t>(ix->RC) * ix->Kr, 0.f);
-    std::vector<float> vals;
-    for (int cb = 0; cb < ix->RC; cb++) {
-        const int j0 = ix->RC == 1 ? 0 : cb * Ds, j1 = ix->RC == 1 ? d : j0 + Ds;
-        vals.resize(static_cast<size_t>(n_train) * (j1 - j0));
-        size_t t = 0;
-        for (int64_t i = 0; i < n_train; i++)
-            for (int j = j0; j < j1; j++) vals[t++] = resid(i, j);
+    // one codebook: the threads share its values; one per subspace: they share
+    // the codebooks
+    const int per = ix->RC == 1 ? d : Ds;  // dimensions of a codebook
+    const unsigned T = n_train * per < (1 << 16) ? 1u : jhq::host_threads();
+    auto train_book = [&](int cb, unsigned threads) {
+        std::vector<float> vals(static_cast<size_t>(n_train) * per);
+        jhq::parallel(threads, [&](unsigned t) {
+            for (int64_t i = n_train * t / threads; i < n_train * (t + 1) / threads; i++)
+                for (int j = 0; j < per; j++)
+                    vals[static_cast<size_t>(i) * per + j] = resid(i, cb * per + j);
+        });
         std::vector<float> c = jhq::train_1d_kmeans(vals.data(), static_cast<int64_t>(vals.size()),
-                                                    ix->Kr);
+                                                    ix->Kr, 25, threads);
         // Kr shrinks only for tiny training sets (train_1d_kmeans clamps Kr to n)
         for (int r = 0; r < ix->Kr; r++)
             ix->res_c1d[static_cast<size_t>(cb) * ix->Kr + r] =
                 c.empty() ? 0.f : c[std::min<size_t>(r, c.size() - 1)];
+    };
+    if (ix->RC == 1) {
+        train_book(0, T);
+    } else {
+        const unsigned Tb = std::min<unsigned>(jhq::host_threads(), static_cast<unsigned>(ix->RC));
+        jhq::parallel(Tb, [&](unsigned t) {
+            for (int cb = static_cast<int>(t); cb < ix->RC; cb += static_cast<int>(Tb)) train_book(cb, 1);
+        });
     }
     JHQ_TRY(ix->dres_c1d.upload(ix->res_c1d.data(), ix->res_c1d.size()));
     JHQ_TRY(build_query_matrix(ix));
@@ -1738,10 +1752,14 @@ int jhq_train(jhq_index* ix, const float* x, int64_t n_train) {
 int jhq_train_ex(jhq_index* ix, const void* x, int dtype, int64_t n_train) {
     if (!ix || !x) return fail(JHQ_EINVAL, "null argument");
     if (n_train <= 0) return fail(JHQ_EINVAL, "n_train must be positive");
-    std::vector<float> tmp;
-    const float* xf = nullptr;
-    JHQ_TRY(host_f32(x, dtype, n_train * static_cast<int64_t>(ix->d), &tmp, &xf));
-    return train_impl(ix, xf, n_train);
+    try {
+        std::vector<float> tmp;
+        const float* xf = nullptr;
+        JHQ_TRY(host_f32(x, dtype, n_train * static_cast<int64_t>(ix->d), &tmp, &xf));
+        return train_impl(ix, xf, n_train);
+    } catch (const std::bad_alloc&) {
+        return fail(JHQ_ENOMEM, "host allocation failed");
+    }
 }
 
 // v14/jhq_gpu_index.cu:417-532
