@@ -62,7 +62,8 @@ typedef struct {
     int   nlist;      /* IVF lists                                     */
     int   nprobe;     /* lists probed per query (clamped to nlist)     */
     int   ivf_iters;  /* Lloyd iterations of the coarse k-means        */
-    int   batch_size; /* queries per search batch                      */
+    int   batch_size; /* queries per search batch (calls with more queries
+                       * may run several of them as one)               */
     int   seed;       /* JL rotation seed                              */
     int   add_batch;  /* rows rotated/encoded per add() step           */
     /* Extension (no reference counterpart; the reference trains one residual
@@ -130,13 +131,15 @@ int jhq_search_ex(jhq_index* idx, const void* q, int dtype, int64_t nq, int k,
  * the workspace reserved for k <= k_max (jhq_reserve; add(), append(),
  * load() and the setters reserve k_max = 10 at the index's batch_size,
  * nprobe and alpha) and fails with JHQ_ESTATE for a larger k.
- * More than batch_size queries: consecutive batches rotate through the
+ * More than batch_size queries: the call runs in batches of a multiple of
+ * batch_size, up to 512 queries as far as the workspace reserved for them
+ * stays small; consecutive batches rotate through the
  * internal search lanes (a workspace and a stream each; of six created, the
  * ones on hardware queues of their own) forked from `stream`
  * and joined back into it, so the call is stream-ordered on `stream` like a
- * single launch; a lane takes two consecutive batches at a time and runs
- * their query product as one launch (each batch's results are those of
- * its own product).  Consecutive device
+ * single launch; with many batches of up to 128 queries a lane takes two at a
+ * time and runs their query product as one launch (each batch's results are
+ * those of its own product).  Consecutive device
  * searches are ordered after each other whatever their streams; add,
  * append, host searches, setters and destroy wait for the last one. */
 int jhq_search_device(jhq_index* idx, const float* d_q, int64_t nq, int k,

@@ -150,6 +150,10 @@ static_assert(kLanes >= 1, "at least one lane");
 #endif
 constexpr int kQbShare = JHQ_QB_SHARE;
 static_assert(kQbShare >= 1, "at least one batch per product");
+// Batches of more than 128 queries keep their own (262 K x 1024 in batches of
+// 128: 2190 us a call on products of their own, 2079 on shared ones; 256: no
+// difference).
+constexpr int qb_share(int batch) { return batch <= 128 ? kQbShare : 1; }
 
 // Per-batch search buffers (v14/search.cuh:24-46).  The index keeps one set
 // per search lane (kLanes): consecutive batches of one device search take the
@@ -163,11 +167,12 @@ struct Workspace {
     DBuf<float> wqpart;
     // integer-MFMA pre-scan: quantized queries and the batch's list hash
     DBuf<unsigned char> wmfma;
-    // the hash in wmfma is clear for batches of hash_P probes at hash_ws
+    // the hash in wmfma is clear for batches of hash_P probes at hash_ws, laid out
+    // for hash_B queries
     // (each batch's re-check clears it for the next; a batch that stopped
     // between its selection and its re-check leaves it unclear)
     bool hash_clear = false;
-    int hash_P = 0;
+    int hash_P = 0, hash_B = 0;
     const unsigned char* hash_ws = nullptr;
 };
 
@@ -194,12 +199,17 @@ struct jhq_index {
     // byte-LUT scans only; 2: the pre-scan wherever it applies
     int scan_kind = 0;
     // the default scan kind's choice of the pre-scan, measured on stored
-    // vectors taken as queries; valid for batches of mfma_dec_B queries with
-    // mfma_dec_P probes while the index holds 0.8 to 1.25 times mfma_dec_n
-    // vectors
-    int mfma_dec_B = 0, mfma_dec_P = 0;
-    int64_t mfma_dec_n = 0;
-    double mfma_dec_cost = 0.0, mfma_dec_cand = 0.0;
+    // vectors taken as queries; valid for batches of B queries with P probes
+    // while the index holds 0.8 to 1.25 times n vectors (one entry for batches
+    // of batch_size queries, one for merged ones)
+    struct MfmaDecision {
+        int B = 0, P = 0;
+        int64_t n = 0;
+        double cost = 0.0, cand = 0.0;
+    } mfma_dec[2];
+    // queries of a batch where a call has more than batch_size (merged_rows);
+    // the workspaces hold this many
+    int bcap = 0;
     // largest per-query candidate count of the dump scan for dump_P probes
     int dump_P = -1;
     int64_t dump_perq = 0;
@@ -563,7 +573,7 @@ int need(DBuf<T>& b, size_t count, bool grow) {
 
 int ensure_workspace(jhq_index* ix, Workspace& w, int ck, int k, int P, int max_segments,
                      bool grow) {
-    const size_t B = static_cast<size_t>(ix->batch_size);
+    const size_t B = static_cast<size_t>(ix->bcap);
     JHQ_TRY(need(w.wq, B * ix->d, grow));
     JHQ_TRY(need(w.wqrot, B * ix->d, grow));
     JHQ_TRY(need(w.wscores, B * ix->nlist, grow));
@@ -576,10 +586,8 @@ int ensure_workspace(jhq_index* ix, Workspace& w, int ck, int k, int P, int max_
     JHQ_TRY(need(w.wout_d, B * k, grow));
     JHQ_TRY(need(w.wout_i, B * k, grow));
     if (ix->dqmat.p) {
-        // split sums for kQbShare batches (a device search's lanes run the
-        // product once for consecutive batches)
-        const size_t pf =
-            jhq::mfma_qb_space(ix->batch_size * kQbShare, ix->d + ix->nlist, ix->d);
+        // split sums of the largest product
+        const size_t pf = jhq::mfma_qb_space(ix->bcap * qb_share(ix->bcap), ix->d + ix->nlist, ix->d);
         if (pf) JHQ_TRY(need(w.wqpart, pf, grow));
     }
     return JHQ_OK;
@@ -689,22 +697,22 @@ int mfma_choose(jhq_index* ix, int Bq, int P, int ck, bool measure, bool* use) {
     }
     if (ck > kMfmaMaxCk || ix->M < kMfmaMinM)
         return JHQ_OK;
-    const int B = ix->batch_size;
-    const bool cached = ix->mfma_dec_B == B && ix->mfma_dec_P == P && ix->mfma_dec_n > 0 &&
-                        ix->ntotal * 5 >= ix->mfma_dec_n * 4 && ix->ntotal * 4 <= ix->mfma_dec_n * 5;
+    auto& dec = ix->mfma_dec[Bq == ix->batch_size ? 0 : 1];
+    const bool cached = dec.B == Bq && dec.P == P && dec.n > 0 && ix->ntotal * 5 >= dec.n * 4 &&
+                        ix->ntotal * 4 <= dec.n * 5;
     if (!cached && measure && ix->ntotal > 0) {
-        JHQ_TRY(mfma_measure_cost(ix, B, P, &ix->mfma_dec_cost, &ix->mfma_dec_cand));
-        ix->mfma_dec_B = B;
-        ix->mfma_dec_P = P;
-        ix->mfma_dec_n = ix->ntotal;
+        JHQ_TRY(mfma_measure_cost(ix, Bq, P, &dec.cost, &dec.cand));
+        dec.B = Bq;
+        dec.P = P;
+        dec.n = ix->ntotal;
         if (verbose())
             std::fprintf(stderr,
                          "[jhq] plan: pre-scan %.2f rows per pair, %.0f candidates per query "
                          "(batch %d, %d probes): %s\n",
-                         ix->mfma_dec_cost, ix->mfma_dec_cand, B, P,
-                         ix->mfma_dec_cost <= kMfmaMaxTileCost ? "pre-scan" : "byte-LUT scan");
+                         dec.cost, dec.cand, Bq, P,
+                         dec.cost <= kMfmaMaxTileCost ? "pre-scan" : "byte-LUT scan");
     }
-    *use = (cached || (measure && ix->ntotal > 0)) && ix->mfma_dec_cost <= kMfmaMaxTileCost;
+    *use = (cached || (measure && ix->ntotal > 0)) && dec.cost <= kMfmaMaxTileCost;
     return JHQ_OK;
 }
 
@@ -785,14 +793,66 @@ int refresh_rows(jhq_index* ix) {
 }
 
 struct BatchPlan {
+    int Bq;    // queries per batch at most
+    int rows;  // queries per batch of the call
     int ck, P;
     jhq::ScanShape sh;
 };
+
+// Candidate slots a query can have at most: the padded sizes of the P largest
+// lists (cached per P; inserts reset the cache).
+int64_t slots_per_query(jhq_index* ix, int P) {
+    if (ix->dump_P != P) {
+        std::vector<int32_t> sz(ix->l_size);
+        std::partial_sort(sz.begin(), sz.begin() + P, sz.end(), std::greater<int32_t>());
+        int64_t per_q = 0;
+        for (int i = 0; i < P; i++)
+            per_q += (sz[i] + jhq::kGroup - 1) / jhq::kGroup * jhq::kGroup;
+        ix->dump_P = P;
+        ix->dump_perq = std::max<int64_t>(per_q, 1);
+    }
+    return ix->dump_perq;
+}
+
+// Queries per batch of a call with more than batch_size of them: as many whole
+// batch_size's as fit in kMergeRows.  A batch is a chain of 4 to 6 launches
+// whose time hardly depends on its queries while they are few, and larger ones
+// share more of their lists, so small batches spend a call on launches and
+// start-up.  Measured in batches of B against 128, 256, 512 and 1024 queries: 1 M
+// x 100 int8, 320 queries, B 32: 584 us, 315, 258, 202, 202; 300 K x 384, k 100,
+// 4000 queries, B 128: 2243, 2212, 1866, 1725, 1735; 262 K x 1024, 4096 queries,
+// B 64: 2200, 1968, 1844 (then the pair limit); 20 K x 96, 37 queries, B 16: 150
+// us, in one batch 88.  Not past the pre-scan's pair limit, the LDS plan,
+// kMergeSlots candidate slots of dump buffer (512 MB of keys) or kMergeScores
+// score floats (128 MB) per lane.
+constexpr int kMergeRows = 512;
+constexpr int64_t kMergeSlots = (int64_t)1 << 26, kMergeScores = (int64_t)1 << 25;
+
+int merged_rows(jhq_index* ix) {
+    const int B = ix->batch_size, P = std::min(ix->nprobe, ix->nlist);
+    const int ck = ceil_ck(ix->alpha, ix->res_k), rck = ix->RC * ix->Kr;
+    const int64_t perq = slots_per_query(ix, P);
+    auto path = [&](int rows, bool* mfma, jhq::ScanShape* sh) {
+        *mfma = jhq::mfma_scan_ok(ix->M, ix->d, ix->Ds, ix->K1D, ix->bpd, rows, P, ck, rck);
+        return jhq::scan_plan(ix->M, ix->d, P, ck, ix->K1D, rows, ix->num_cu, sh, skew_eligible(ix),
+                              false, rck);
+    };
+    bool m0, m1;
+    jhq::ScanShape s0{}, s1{};
+    if (B >= kMergeRows || !path(B, &m0, &s0)) return B;
+    for (int rows = kMergeRows / B * B; rows > B; rows -= B)
+        if (rows * perq <= kMergeSlots &&
+            static_cast<int64_t>(rows) * (ix->d + ix->nlist) <= kMergeScores && path(rows, &m1, &s1) && m1 == m0 && s1.wave == s0.wave &&
+            s1.skew == s0.skew && s1.dump == s0.dump)
+            return rows;
+    return B;
+}
 
 // The plan of a search batch and the workspaces it needs on nws lanes.
 // grow = false (device searches): nothing is allocated or refreshed, and a
 // shape beyond the reservation fails with JHQ_ESTATE.
 int plan_batch(jhq_index* ix, int Bq, int k, BatchPlan* bp, int nws, bool grow) {
+    bp->Bq = bp->rows = Bq;
     bp->ck = ceil_ck(ix->alpha, k);
     bp->P = std::min(ix->nprobe, ix->nlist);
     bool use_mfma = false;
@@ -813,30 +873,19 @@ int plan_batch(jhq_index* ix, int Bq, int k, BatchPlan* bp, int nws, bool grow) 
     for (int i = 0; i < nws; i++)
         JHQ_TRY(ensure_workspace(ix, ix->ws[i], bp->ck, k, bp->P, bp->sh.max_segments, grow));
     if (bp->sh.dump || bp->sh.mfma) {
-        // a query's candidates are at most the padded sizes of the P largest
-        // lists (cached per P; inserts reset the cache)
-        if (ix->dump_P != bp->P) {
-            std::vector<int32_t> sz(ix->l_size);
-            std::partial_sort(sz.begin(), sz.begin() + bp->P, sz.end(), std::greater<int32_t>());
-            int64_t per_q = 0;
-            for (int i = 0; i < bp->P; i++)
-                per_q += (sz[i] + jhq::kGroup - 1) / jhq::kGroup * jhq::kGroup;
-            ix->dump_P = bp->P;
-            ix->dump_perq = per_q;
-        }
         // keys (dump scan) or biased integer distances (MFMA pre-scan)
         // (the pre-scan: u32 slots and one tile minimum per 16 after them)
         // (grown with an eighth to spare: appends lengthen the lists a little
         // at a time, and each reallocation here is one per lane)
-        const size_t slots = static_cast<size_t>(Bq) * std::max<int64_t>(ix->dump_perq, 1);
+        const size_t slots = static_cast<size_t>(ix->bcap) * slots_per_query(ix, bp->P);
         const size_t words = bp->sh.mfma ? (slots + slots / 16 + 40) / 2 : slots;
         for (int i = 0; i < nws; i++)
             if (!ix->ws[i].wdump.has(words))
                 JHQ_TRY(need(ix->ws[i].wdump, grow ? words + words / 8 : words, grow));
         if (bp->sh.mfma)
             for (int i = 0; i < nws; i++)
-                JHQ_TRY(need(ix->ws[i].wmfma, jhq::mfma_scan_bytes(Bq, bp->P, ix->M, ix->num_cu),
-                             grow));
+                JHQ_TRY(need(ix->ws[i].wmfma,
+                             jhq::mfma_scan_bytes(ix->bcap, bp->P, ix->M, ix->num_cu), grow));
     }
     return JHQ_OK;
 }
@@ -863,12 +912,13 @@ int run_batch(jhq_index* ix, Workspace& w, const float* d_q, int Bq, int k, cons
     // batch's (query, probe) pairs in the workspace's list hash
     const int64_t dump_slots = static_cast<int64_t>(w.wdump.n * 2 / 17 * 16);
     jhq::PrescanSel ps{w.wmfma.p, w.wmfma.n, dump_slots, w.wqrot.p, ix->dc1d.p, d, ix->M,
-                       ix->batch_size};
+                       bp.Bq};
     if (bp.sh.mfma) {
-        if (!w.hash_clear || w.hash_P != bp.P || w.hash_ws != w.wmfma.p)
-            JHQ_HIP(jhq::mfma_hash_clear(ix->batch_size, bp.P, ix->M, w.wmfma.p, w.wmfma.n, s));
+        if (!w.hash_clear || w.hash_P != bp.P || w.hash_B != bp.Bq || w.hash_ws != w.wmfma.p)
+            JHQ_HIP(jhq::mfma_hash_clear(bp.Bq, bp.P, ix->M, w.wmfma.p, w.wmfma.n, s));
         w.hash_clear = false;
         w.hash_P = bp.P;
+        w.hash_B = bp.Bq;
         w.hash_ws = w.wmfma.p;
     }
     if (ix->dqmat.p) {
@@ -907,7 +957,7 @@ int run_batch(jhq_index* ix, Workspace& w, const float* d_q, int Bq, int k, cons
                                dump_slots, w.wmfma.p, w.wmfma.n, k, ix->dres_c1d.p, ix->Kr,
                                ix->RC, ix->Br, ix->bpv, ix->dres.p, ix->dcorr.p,
                                ix->dlist_ids.p, d_out, d_ids, want_topck ? w.wtopck.p : nullptr,
-                               w.wpartial.p, w.wpslot.p, ix->num_cu, ix->batch_size, s));
+                               w.wpartial.p, w.wpslot.p, ix->num_cu, bp.Bq, s));
         // the re-check clears the hash for the lane's next batch
         w.hash_clear = true;
         if (ix->timing) JHQ_HIP(hipEventRecord(ix->ev[3], s));
@@ -968,11 +1018,11 @@ int ensure_host_staging(jhq_index* ix, int l, int Bmax, int k) {
 bool skew_needed(jhq_index* ix) {
     if (!skew_eligible(ix)) return false;
     const int P = std::min(ix->nprobe, ix->nlist);
-    for (int k = 1; k <= ix->res_k; k++) {
-        bool mf = false;
-        if (mfma_choose(ix, ix->batch_size, P, ceil_ck(ix->alpha, k), true, &mf) != JHQ_OK || !mf)
-            return true;
-    }
+    for (int B : {ix->batch_size, ix->bcap})
+        for (int k = 1; k <= ix->res_k; k++) {
+            bool mf = false;
+            if (mfma_choose(ix, B, P, ceil_ck(ix->alpha, k), true, &mf) != JHQ_OK || !mf) return true;
+        }
     return false;
 }
 
@@ -988,27 +1038,58 @@ int reserve_search(jhq_index* ix) {
     // insert's enqueued tail does not read them; the refreshes below are
     // enqueued behind it)
     JHQ_TRY(ix->quiesce_searches());
+    ix->bcap = merged_rows(ix);
     if (ix->skew_stale && skew_needed(ix)) JHQ_TRY(refresh_skew(ix));
     if (rows_wanted(ix) && ix->rows_stale) JHQ_TRY(refresh_rows(ix));
+    // the plans of the longest short list, of the shortest, and of the longest
+    // that may take the pre-scan, for both batch sizes
+    int kpre = ix->res_k;
+    while (kpre > 1 && ceil_ck(ix->alpha, kpre) > kMfmaMaxCk) kpre--;
     BatchPlan bp;
-    JHQ_TRY(plan_batch(ix, ix->batch_size, ix->res_k, &bp, kLanes, true));
+    for (int k : {ix->res_k, kpre, 1}) {
+        JHQ_TRY(plan_batch(ix, ix->batch_size, k, &bp, kLanes, true));
+        if (ix->bcap > ix->batch_size) JHQ_TRY(plan_batch(ix, ix->bcap, k, &bp, kLanes, true));
+    }
     JHQ_TRY(ix->ensure_lanes());
-    for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, ix->batch_size, ix->res_k));
+    for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, ix->bcap, ix->res_k));
     return JHQ_OK;
+}
+
+// The plan of a call of nq queries: batches of batch_size, or, past that, of
+// bcap where a plan of that size exists.  Host calls (grow) with more than
+// kHostChunk bytes of queries go in up to four batches, so that the copies of
+// one run beside the kernels of another (1000 x 768: 375 us in batches of 256,
+// 423 in 512; 264 x 384 in one batch 143 us, in four 207).
+constexpr int64_t kHostChunk = (int64_t)512 << 10;
+
+int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan* bp, bool* pipe) {
+    if (grow) ix->bcap = merged_rows(ix);
+    int rows = ix->bcap;
+    if (grow) {
+        const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(4, nq * ix->d * 4 / kHostChunk));
+        rows = static_cast<int>(std::min<int64_t>(rows, (nq + parts - 1) / parts));
+    }
+    if (merge && nq > ix->batch_size && rows > ix->batch_size &&
+        plan_batch(ix, ix->bcap, k, bp, nq > rows ? kLanes : 1, grow) == JHQ_OK) {
+        bp->rows = rows;
+        *pipe = nq > rows;
+        return JHQ_OK;
+    }
+    *pipe = merge && nq > ix->batch_size;
+    return plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
 }
 
 // Host arrays over several batches: the batches rotate through the lanes
 // (workspace, pinned staging, stream).  While the other lanes' batches run,
 // the host copies a lane's finished results out and its next queries in.
-int search_host_pipelined(jhq_index* ix, const float* q, int64_t nq, int k, float* dists,
-                          int32_t* ids) {
+int search_host_pipelined(jhq_index* ix, const float* q, int64_t nq, int k, const BatchPlan& bp,
+                          float* dists, int32_t* ids) {
     const int d = ix->d;
-    const int Bmax = ix->batch_size;
-    BatchPlan bp;
-    JHQ_TRY(plan_batch(ix, Bmax, k, &bp, kLanes, true));
+    const int Bmax = bp.rows;
     JHQ_TRY(ix->ensure_lanes());
     for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, Bmax, k));
-    const int nl = ix->nlanes;
+    // (the lanes that get a batch)
+    const int nl = static_cast<int>(std::min<int64_t>(ix->nlanes, (nq + Bmax - 1) / Bmax));
     JHQ_HIP(hipEventRecord(ix->lane_ev[0], ix->stream));
     for (int i = 0; i < nl; i++)
         JHQ_HIP(hipStreamWaitEvent(ix->lane[ix->lane_use[i]], ix->lane_ev[0], 0));
@@ -1059,11 +1140,12 @@ int search_host(jhq_index* ix, const float* q, int64_t nq, int k, float* dists, 
     // a device search may still use the workspaces, which a larger k regrows
     JHQ_TRY(ix->quiesce());
     const int d = ix->d;
-    const int Bmax = ix->batch_size;
     const bool dbg = (q_rot || probes || topck_pos || topck_dist);
-    if (!dbg && !ix->timing && nq > Bmax) return search_host_pipelined(ix, q, nq, k, dists, ids);
     BatchPlan bp;
-    JHQ_TRY(plan_batch(ix, Bmax, k, &bp, 1, true));
+    bool pipe = false;
+    JHQ_TRY(plan_call(ix, nq, k, true, !dbg && !ix->timing, &bp, &pipe));
+    if (pipe) return search_host_pipelined(ix, q, nq, k, bp, dists, ids);
+    const int Bmax = bp.rows;
     JHQ_TRY(ensure_host_staging(ix, 0, Bmax, k));
     std::vector<unsigned long long> tk;
     for (int64_t q0 = 0; q0 < nq; q0 += Bmax) {
@@ -1168,6 +1250,7 @@ int jhq_create(int d, const jhq_params* p, jhq_index** out) {
     ix->nprobe = std::min(p->nprobe, p->nlist);
     ix->ivf_iters = p->ivf_iters;
     ix->batch_size = p->batch_size;
+    ix->bcap = p->batch_size;
     ix->seed = p->seed;
     ix->add_batch = p->add_batch;
     ix->alpha = p->alpha;
@@ -1806,15 +1889,14 @@ int jhq_search_device(jhq_index* ix, const float* d_q, int64_t nq, int k, float*
     if (!d_q || !d_dists || !d_ids) return fail(JHQ_EINVAL, "null argument");
     if (nq == 0) return JHQ_OK;
     hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ix->stream;
-    const int Bmax = ix->batch_size;
     // several batches: rotate through the search lanes (workspace and stream
     // each), forked from s and joined back into it (step timing keeps one
-    // stream)
-    const bool pipe = nq > Bmax && !ix->timing;
-    // enqueue-only: the reserved workspace must cover this shape (no
+    // stream).  Enqueue-only: the reserved workspace must cover this shape (no
     // allocation, no host synchronisation)
     BatchPlan bp;
-    JHQ_TRY(plan_batch(ix, Bmax, k, &bp, pipe ? kLanes : 1, false));
+    bool pipe = false;
+    JHQ_TRY(plan_call(ix, nq, k, false, !ix->timing, &bp, &pipe));
+    const int Bmax = bp.rows;
     if (pipe && !ix->lane[kLanes - 1])
         return fail(JHQ_ESTATE, "search lanes are not set up; call jhq_reserve()");
     // ordered after the previous device search (it shares the workspaces),
@@ -1832,20 +1914,23 @@ int jhq_search_device(jhq_index* ix, const float* d_q, int64_t nq, int k, float*
         ix->done_pending = true;
         return JHQ_OK;
     }
-    const int nl = ix->nlanes;
+    // consecutive batches share their lane's query product where the
+    // selection adds its split sums and every lane has batches enough
+    const int d = ix->d;
+    const int64_t nb = (nq + Bmax - 1) / Bmax;
+    const int group = qb_share(Bmax);
+    const bool share = group > 1 && ix->dqmat.p && nb >= 2 * group * ix->nlanes &&
+                       jhq::select_adds_qb(jhq::mfma_qb_plan(Bmax * group, d + ix->nlist, d),
+                                           ix->nlist, d);
+    // (the lanes that get a batch)
+    const int nl = static_cast<int>(std::min<int64_t>(ix->nlanes, nb));
     JHQ_HIP(hipEventRecord(ix->lane_ev[0], s));
     for (int i = 0; i < nl; i++)
         JHQ_HIP(hipStreamWaitEvent(ix->lane[ix->lane_use[i]], ix->lane_ev[0], 0));
-    // consecutive batches share their lane's query product where the
-    // selection adds its split sums
-    const int d = ix->d;
-    const bool share = kQbShare > 1 && ix->dqmat.p &&
-                       jhq::select_adds_qb(jhq::mfma_qb_plan(Bmax * kQbShare, d + ix->nlist, d),
-                                           ix->nlist, d);
     int64_t bi = 0;
     for (int64_t q0 = 0; q0 < nq; bi++) {
         const int l = ix->lane_use[bi % nl];
-        const int64_t rows = std::min<int64_t>(static_cast<int64_t>(Bmax) * (share ? kQbShare : 1),
+        const int64_t rows = std::min<int64_t>(static_cast<int64_t>(Bmax) * (share ? group : 1),
                                                nq - q0);
         // one batch alone keeps its own product
         const int srows = rows > Bmax ? static_cast<int>(rows) : 0;
