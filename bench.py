@@ -10,11 +10,11 @@ Default run (the driver's `python bench.py --gpus 1 --steps K --warmup W`):
   first 100,000 base vectors (the reference demo's protocol), M=128, B=8,
   Br=4, k=10, query batch 64.  Ground truth is exact L2 brute force.  A
   "step" is one device search call over the 10,000 queries, resident in HBM
-  with their results: the engine runs them in batches of 64 through the whole
+  with their results: the index's batch size is 64, and the engine runs a
+  call of more queries in merged batches of a multiple of it through the whole
   search path, consecutive batches on the search lanes that have hardware
   queues of their own (four of six streams; forked from and joined into the
-  caller's stream; a lane takes two consecutive batches at a time, with one
-  query-product launch for both).  The sweep nprobe {16, 32, 64} x
+  caller's stream).  The sweep nprobe {16, 32, 64} x
   alpha {4, 10} picks the fastest point with recall@10 >= 0.95; when no point
   reaches it (the codes' own recall ceiling, measured by ranking every vector
   by its full estimate, is below 0.95 on this data) the fastest point within
@@ -662,7 +662,9 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
         "frac": round(max(f_hbm, f_mfma), 4),
         "traffic": traffic,
         "time_base": "us per batch in the timed pipelined run: HIP events on the caller's "
-                     "stream around the timed steps / batches per step",
+                     "stream around the timed steps / batches of batch_size per step (bytes and "
+                     "ops counted per such batch; the engine merges batches, which read "
+                     "fewer of their shared lists than this counts)",
         "us_per_batch_pipelined": round(t_batch, 2),
         "algorithmic_bytes_per_batch": int(step_bytes),
         "bytes_breakdown": {k2: int(v) for k2, v in parts.items()},

@@ -1026,19 +1026,8 @@ bool skew_needed(jhq_index* ix) {
     return false;
 }
 
-// Preallocates everything a search with k <= res_k needs (the reference's
-// alloc_workspace at the end of add(), v14/jhq_gpu_index.cu:166-206,531, and
-// realloc_ck_buffers, v14/search.cu:294-313): every lane's workspace, stream
-// and pinned staging, and an up-to-date skewed code copy.  Called after every
-// add / append / load and parameter change, so device searches allocate
-// nothing.
-int reserve_search(jhq_index* ix) {
-    if (ix->ntotal == 0 || !ix->trained) return JHQ_OK;
-    // workspaces may be regrown: no device search may be using them (an
-    // insert's enqueued tail does not read them; the refreshes below are
-    // enqueued behind it)
-    JHQ_TRY(ix->quiesce_searches());
-    ix->bcap = merged_rows(ix);
+// The copies, workspaces, lanes and staging of batches of up to bcap queries.
+int reserve_batches(jhq_index* ix) {
     if (ix->skew_stale && skew_needed(ix)) JHQ_TRY(refresh_skew(ix));
     if (rows_wanted(ix) && ix->rows_stale) JHQ_TRY(refresh_rows(ix));
     // the plans of the longest short list, of the shortest, and of the longest
@@ -1055,6 +1044,37 @@ int reserve_search(jhq_index* ix) {
     return JHQ_OK;
 }
 
+// After a failed allocation: merged batches are not worth failing for (their
+// workspaces are several times those of batch_size queries), so they are off
+// until the next reservation.  True if there is a smaller size to go on with.
+bool drop_merged(jhq_index* ix, int rc) {
+    if (rc != JHQ_ENOMEM || ix->bcap <= ix->batch_size) return false;
+    (void)hipGetLastError();  // launches would report the allocation's error
+    ix->bcap = ix->batch_size;
+    return true;
+}
+
+// Preallocates everything a search with k <= res_k needs (the reference's
+// alloc_workspace at the end of add(), v14/jhq_gpu_index.cu:166-206,531, and
+// realloc_ck_buffers, v14/search.cu:294-313): every lane's workspace, stream
+// and pinned staging, and an up-to-date skewed code copy.  Called after every
+// add / append / load and parameter change, so device searches allocate
+// nothing.
+int reserve_search(jhq_index* ix) {
+    if (ix->ntotal == 0 || !ix->trained) return JHQ_OK;
+    // workspaces may be regrown: no device search may be using them (an
+    // insert's enqueued tail does not read them; the refreshes are enqueued
+    // behind it)
+    JHQ_TRY(ix->quiesce_searches());
+    const int prev = ix->bcap;
+    ix->bcap = merged_rows(ix);
+    int rc = reserve_batches(ix);
+    if (drop_merged(ix, rc)) rc = reserve_batches(ix);
+    // the caller goes back to the settings that the workspaces are sized for
+    if (rc != JHQ_OK) ix->bcap = prev;
+    return rc;
+}
+
 // The plan of a call of nq queries: batches of batch_size, or, past that, of
 // bcap where a plan of that size exists.  Host calls (grow) with more than
 // kHostChunk bytes of queries go in up to four batches, so that the copies of
@@ -1063,19 +1083,23 @@ int reserve_search(jhq_index* ix) {
 constexpr int64_t kHostChunk = (int64_t)512 << 10;
 
 int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan* bp, bool* pipe) {
-    if (grow) ix->bcap = merged_rows(ix);
     int rows = ix->bcap;
     if (grow) {
         const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(4, nq * ix->d * 4 / kHostChunk));
         rows = static_cast<int>(std::min<int64_t>(rows, (nq + parts - 1) / parts));
     }
-    if (merge && nq > ix->batch_size && rows > ix->batch_size &&
-        plan_batch(ix, ix->bcap, k, bp, nq > rows ? kLanes : 1, grow) == JHQ_OK) {
-        bp->rows = rows;
-        *pipe = nq > rows;
-        return JHQ_OK;
+    if (merge && nq > ix->batch_size && rows > ix->batch_size) {
+        const int rc = plan_batch(ix, ix->bcap, k, bp, nq > rows ? kLanes : 1, grow);
+        if (rc == JHQ_OK) {
+            bp->rows = rows;
+            *pipe = nq > rows;
+            return JHQ_OK;
+        }
+        if (grow) (void)drop_merged(ix, rc);
     }
     *pipe = merge && nq > ix->batch_size;
+    const int rc = plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
+    if (!grow || !drop_merged(ix, rc)) return rc;
     return plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
 }
 

@@ -1,0 +1,61 @@
+"""Search calls with more queries than batch_size run in merged batches of up
+to 512 queries: the ids and distances of every call are, bit for bit, those of
+one call per batch_size queries (host and device, each scan kind, sizes around
+the merged batch, the lanes and a ragged last batch)."""
+import numpy as np
+import pytest
+
+import jhq_gpu_amd as jg
+
+pytestmark = pytest.mark.gpu
+
+# d, M, Br, nlist, nprobe, batch, alpha, k
+SHAPES = {
+    "one_bit_prescan": (128, 16, 4, 24, 6, 16, 4.0, 10),
+    "two_bit": (100, 25, 4, 24, 5, 32, 4.0, 10),
+    "flat": (96, 12, 8, 1, 1, 7, 4.0, 1),
+    "long_lists": (128, 32, 4, 16, 16, 100, 4.0, 100),
+    "batch_over_512": (64, 16, 4, 16, 4, 600, 4.0, 10),
+}
+
+
+@pytest.fixture(scope="module", params=sorted(SHAPES))
+def built(request, gpu):
+    d, M, Br, nlist, nprobe, batch, alpha, k = SHAPES[request.param]
+    g = np.random.default_rng(5)
+    x = g.standard_normal((6000, d)).astype(np.float32)
+    ix = jg.JHQGpuIndex(d, jg.Params(M=M, B=8, Br=Br, alpha=alpha, nlist=nlist, nprobe=nprobe,
+                                     ivf_iters=2, batch_size=batch, seed=42))
+    ix.train(x[:3000])
+    ix.add(x)
+    ix.reserve(k)
+    q = g.standard_normal((2100, d)).astype(np.float32)
+    return ix, q, batch, k
+
+
+def _bits(a):
+    return np.ascontiguousarray(a).view(np.uint32)
+
+
+@pytest.mark.parametrize("kind", [0, 1, 2])
+def test_merged_batches_equal_single_ones(built, gpu, kind):
+    import torch
+    ix, q, B, k = built
+    ix.set_scan_kind(kind)
+    try:
+        parts = [ix.search(q[i:i + B], k) for i in range(0, len(q), B)]
+        want_d = np.concatenate([p[0] for p in parts])
+        want_i = np.concatenate([p[1] for p in parts])
+        for nq in sorted({B, B + 1, 511, 512, 513, 1029, 2100}):
+            d, i = ix.search(q[:nq], k)
+            assert np.array_equal(i, want_i[:nq]), nq
+            assert np.array_equal(_bits(d), _bits(want_d[:nq])), nq
+            qt = torch.from_numpy(q[:nq]).to(gpu)
+            od = torch.full((nq, k), -1.0, device=gpu)
+            oi = torch.full((nq, k), -2, dtype=torch.int32, device=gpu)
+            for _ in range(2):
+                ix.search_device(qt, k, od, oi, stream=torch.cuda.current_stream())
+            assert np.array_equal(oi.cpu().numpy(), want_i[:nq]), nq
+            assert np.array_equal(_bits(od.cpu().numpy()), _bits(want_d[:nq])), nq
+    finally:
+        ix.set_scan_kind(0)
