@@ -8,7 +8,6 @@
 #include <algorithm>
 #include <cstdint>
 #include <exception>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -54,7 +53,7 @@ void parallel(unsigned T, F f) {
     unsigned started = 1;
     try {
         for (; started < T; started++) th.emplace_back(call, started);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // no thread, or no memory for its state
     }
     call(0);
     for (unsigned t = started; t < T; t++) call(t);
