@@ -12,6 +12,8 @@ pytestmark = pytest.mark.gpu
 # d, M, Br, nlist, nprobe, batch, alpha, k
 SHAPES = {
     "one_bit_prescan": (128, 16, 4, 24, 6, 16, 4.0, 10),
+    # merged calls past the pre-scan's pair limit where it is not the scan
+    "one_bit_many_probes": (128, 16, 4, 80, 70, 32, 4.0, 10),
     "two_bit": (100, 25, 4, 24, 5, 32, 4.0, 10),
     "flat": (96, 12, 8, 1, 1, 7, 4.0, 1),
     "long_lists": (128, 32, 4, 16, 16, 100, 4.0, 100),
