@@ -236,6 +236,12 @@ int jhq_search_debug(jhq_index* idx, const float* q, int64_t nq, int k,
                      float* dists, int32_t* ids, float* q_rot, int32_t* probes,
                      int32_t* topck_pos, float* topck_dist);
 
+/* For tests of memory shortage: of the device buffers of min_bytes <= size <
+ * max_bytes that this thread's calls ask for from now on, the first `skip`
+ * are allocated and the next `count` fail as hipMalloc fails.  Returns how
+ * many failed since the last call (count 0: none fail any more). */
+int64_t jhq_debug_fail_alloc(int64_t min_bytes, int64_t max_bytes, int64_t skip, int64_t count);
+
 /* Per-step device timing (hipEvents around each step, the reference's
  * step list of jhq_v13_step_timing/search.cu:424-491).  When enabled,
  * every search batch records events; jhq_get_timing returns accumulated

@@ -107,6 +107,7 @@ _SIGS = {
     "jhq_get_codebooks": (_I, [_VP, _VP, _VP, _VP, _VP, _VP, _VP]),
     "jhq_get_lists": (_I, [_VP, _VP, _VP, _VP, _VP, _VP]),
     "jhq_search_debug": (_I, [_VP, _VP, _I64, _I, _VP, _VP, _VP, _VP, _VP, _VP]),
+    "jhq_debug_fail_alloc": (_I64, [_I64, _I64, _I64, _I64]),
     "jhq_set_timing": (_I, [_VP, _I]),
     "jhq_get_timing": (_I, [_VP, _VP, _I, ctypes.POINTER(_I64)]),
     "jhq_k_rotate": (_I, [_VP, _VP, _I64, _I, _VP, _VP]),

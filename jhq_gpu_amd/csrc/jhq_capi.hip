@@ -38,12 +38,17 @@ int fail(int code, const std::string& msg) {
     return code;
 }
 
+// A failed HIP call also stays HIP's last error, which the next kernel launch
+// would report as its own: once reported here it is cleared, so that a caller
+// with another way on (a smaller batch, no optional copy) can take it.
 #define JHQ_HIP(expr)                                                                  \
     do {                                                                               \
         hipError_t e_ = (expr);                                                        \
-        if (e_ != hipSuccess)                                                          \
+        if (e_ != hipSuccess) {                                                        \
+            (void)hipGetLastError();                                                   \
             return fail(e_ == hipErrorOutOfMemory ? JHQ_ENOMEM : JHQ_EDEVICE,          \
                         std::string(#expr) + ": " + hipGetErrorString(e_));            \
+        }                                                                              \
     } while (0)
 
 #define JHQ_TRY(expr)            \
@@ -51,6 +56,23 @@ int fail(int code, const std::string& msg) {
         int rc_ = (expr);        \
         if (rc_ != JHQ_OK) return rc_; \
     } while (0)
+
+// Device buffers that this thread's next calls do not get (jhq_debug_fail_alloc).
+struct RefusedAllocs {
+    size_t lo = 0, hi = 0;
+    int64_t skip = 0, count = 0, refused = 0;
+    bool refuse(size_t bytes) {
+        if (count <= 0 || bytes < lo || bytes >= hi) return false;
+        if (skip > 0) {
+            skip--;
+            return false;
+        }
+        count--;
+        refused++;
+        return true;
+    }
+};
+thread_local RefusedAllocs g_refused;
 
 // Owning device buffer.
 template <class T>
@@ -71,10 +93,14 @@ struct DBuf {
     int alloc(size_t count) {
         if (count == 0) count = 1;
         T* np = nullptr;
-        hipError_t e = hipMalloc(reinterpret_cast<void**>(&np), count * sizeof(T));
-        if (e != hipSuccess)
+        // (a refused one asks for more than any device has, so that HIP fails it)
+        const size_t ask = g_refused.refuse(count * sizeof(T)) ? size_t(1) << 60 : count * sizeof(T);
+        hipError_t e = hipMalloc(reinterpret_cast<void**>(&np), ask);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();  // (as in JHQ_HIP)
             return fail(JHQ_ENOMEM, "hipMalloc of " + std::to_string(count * sizeof(T)) +
                                         " bytes: " + hipGetErrorString(e));
+        }
         release();
         p = np;
         n = count;
@@ -1052,7 +1078,6 @@ int reserve_batches(jhq_index* ix) {
 // until the next reservation.  True if there is a smaller size to go on with.
 bool drop_merged(jhq_index* ix, int rc) {
     if (rc != JHQ_ENOMEM || ix->bcap <= ix->batch_size) return false;
-    (void)hipGetLastError();  // launches would report the allocation's error
     ix->bcap = ix->batch_size;
     return true;
 }
@@ -2310,6 +2335,16 @@ int jhq_search_ex(jhq_index* idx, const void* q, int dtype, int64_t nq, int k, f
     const float* qf = nullptr;
     JHQ_TRY(host_f32(q, dtype, nq * static_cast<int64_t>(idx->d), &tmp, &qf));
     return search_host(idx, qf, nq, k, dists, ids, nullptr, nullptr, nullptr, nullptr);
+}
+
+int64_t jhq_debug_fail_alloc(int64_t min_bytes, int64_t max_bytes, int64_t skip, int64_t count) {
+    const int64_t refused = g_refused.refused;
+    g_refused = RefusedAllocs{};
+    g_refused.lo = static_cast<size_t>(std::max<int64_t>(min_bytes, 0));
+    g_refused.hi = static_cast<size_t>(std::max<int64_t>(max_bytes, 0));
+    g_refused.skip = skip;
+    g_refused.count = count;
+    return refused;
 }
 
 int jhq_set_timing(jhq_index* idx, int enable) {
