@@ -200,6 +200,14 @@ struct Workspace {
     bool hash_clear = false;
     int hash_P = 0, hash_B = 0;
     const unsigned char* hash_ws = nullptr;
+    void release() {
+        wq.release(); wqrot.release(); wscores.release(); wout_d.release();
+        wprobes.release(); wgofs.release(); wqtot.release(); wout_i.release(); wpslot.release();
+        wpartial.release(); wtopck.release(); wdump.release();
+        wqpart.release();
+        wmfma.release();
+        hash_clear = false;
+    }
 };
 
 }  // namespace
@@ -236,6 +244,11 @@ struct jhq_index {
     // queries of a batch where a call has more than batch_size (merged_rows);
     // the workspaces hold this many
     int bcap = 0;
+    // the most queries the workspaces were grown for since their last release
+    int ws_rows = 0;
+    // device memory did not do for merged batches: inserts and searches do not
+    // try again, jhq_reserve() and the setters do
+    bool merge_short = false;
     // largest per-query candidate count of the dump scan for dump_P probes
     int dump_P = -1;
     int64_t dump_perq = 0;
@@ -600,6 +613,7 @@ int need(DBuf<T>& b, size_t count, bool grow) {
 int ensure_workspace(jhq_index* ix, Workspace& w, int ck, int k, int P, int max_segments,
                      bool grow) {
     const size_t B = static_cast<size_t>(ix->bcap);
+    if (grow) ix->ws_rows = std::max(ix->ws_rows, ix->bcap);
     JHQ_TRY(need(w.wq, B * ix->d, grow));
     JHQ_TRY(need(w.wqrot, B * ix->d, grow));
     JHQ_TRY(need(w.wscores, B * ix->nlist, grow));
@@ -1075,10 +1089,15 @@ int reserve_batches(jhq_index* ix) {
 
 // After a failed allocation: merged batches are not worth failing for (their
 // workspaces are several times those of batch_size queries), so they are off
-// until the next reservation.  True if there is a smaller size to go on with.
+// and what the workspaces hold goes back to the device.  True if there was
+// anything: the caller tries again, and reserves what it needs afresh.  No
+// search may be in flight.
 bool drop_merged(jhq_index* ix, int rc) {
-    if (rc != JHQ_ENOMEM || ix->bcap <= ix->batch_size) return false;
+    if (rc != JHQ_ENOMEM || ix->ws_rows <= ix->batch_size) return false;
     ix->bcap = ix->batch_size;
+    ix->ws_rows = 0;
+    ix->merge_short = true;
+    for (Workspace& w : ix->ws) w.release();
     return true;
 }
 
@@ -1095,11 +1114,28 @@ int reserve_search(jhq_index* ix) {
     // behind it)
     JHQ_TRY(ix->quiesce_searches());
     const int prev = ix->bcap;
-    ix->bcap = merged_rows(ix);
-    int rc = reserve_batches(ix);
-    if (drop_merged(ix, rc)) rc = reserve_batches(ix);
+    ix->bcap = ix->merge_short ? ix->batch_size : merged_rows(ix);
+    const int rc = reserve_batches(ix);
+    if (drop_merged(ix, rc)) return reserve_batches(ix);
     // the caller goes back to the settings that the workspaces are sized for
     if (rc != JHQ_OK) ix->bcap = prev;
+    return rc;
+}
+
+// A new value of a search setting, with the workspace reserved for it; where
+// that fails, the old value with its reservation.
+template <class T>
+int set_and_reserve(jhq_index* ix, T jhq_index::*field, T value) {
+    const T prev = ix->*field;
+    ix->*field = value;
+    ix->merge_short = false;
+    const int rc = reserve_search(ix);
+    if (rc == JHQ_OK) return rc;
+    ix->*field = prev;
+    const std::string why = g_err;
+    // (the failed attempt may have given merged batches' buffers back)
+    (void)reserve_search(ix);
+    g_err = why;
     return rc;
 }
 
@@ -1123,11 +1159,12 @@ int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan
             *pipe = nq > rows;
             return JHQ_OK;
         }
-        if (grow) (void)drop_merged(ix, rc);
+        if (grow && drop_merged(ix, rc)) (void)reserve_batches(ix);
     }
     *pipe = merge && nq > ix->batch_size;
     const int rc = plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
     if (!grow || !drop_merged(ix, rc)) return rc;
+    (void)reserve_batches(ix);
     return plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
 }
 
@@ -1338,45 +1375,27 @@ int jhq_set_nprobe(jhq_index* idx, int nprobe) {
     if (!idx) return fail(JHQ_EINVAL, "null index");
     if (nprobe <= 0) return fail(JHQ_EINVAL, "nprobe must be positive");
     JHQ_TRY(idx->quiesce());
-    const int prev = idx->nprobe;
-    idx->nprobe = std::min(nprobe, idx->nlist);
-    const int rc = reserve_search(idx);
-    // a failed reservation keeps the setting the workspace was reserved for
-    // (buffers only grow, so that reservation still holds)
-    if (rc != JHQ_OK) idx->nprobe = prev;
-    return rc;
+    return set_and_reserve(idx, &jhq_index::nprobe, std::min(nprobe, idx->nlist));
 }
 
 int jhq_set_alpha(jhq_index* idx, float alpha) {
     if (!idx) return fail(JHQ_EINVAL, "null index");
     if (!(alpha > 0.0f)) return fail(JHQ_EINVAL, "alpha must be positive");
     JHQ_TRY(idx->quiesce());
-    const float prev = idx->alpha;
-    idx->alpha = alpha;
-    const int rc = reserve_search(idx);
-    if (rc != JHQ_OK) idx->alpha = prev;
-    return rc;
+    return set_and_reserve(idx, &jhq_index::alpha, alpha);
 }
 
 int jhq_reserve(jhq_index* idx, int k_max) {
     if (!idx) return fail(JHQ_EINVAL, "null index");
     if (k_max <= 0) return fail(JHQ_EINVAL, "k_max must be positive");
-    const int prev = idx->res_k;
-    idx->res_k = std::max(idx->res_k, k_max);
-    const int rc = reserve_search(idx);
-    if (rc != JHQ_OK) idx->res_k = prev;
-    return rc;
+    return set_and_reserve(idx, &jhq_index::res_k, std::max(idx->res_k, k_max));
 }
 
 int jhq_set_scan_kind(jhq_index* idx, int kind) {
     if (!idx) return fail(JHQ_EINVAL, "null index");
     if (kind < 0 || kind > 2) return fail(JHQ_EINVAL, "scan kind must be 0, 1 or 2");
     JHQ_TRY(idx->quiesce());
-    const int prev = idx->scan_kind;
-    idx->scan_kind = kind;
-    const int rc = reserve_search(idx);
-    if (rc != JHQ_OK) idx->scan_kind = prev;
-    return rc;
+    return set_and_reserve(idx, &jhq_index::scan_kind, kind);
 }
 
 int jhq_get_dims(const jhq_index* idx, int* Ds, int* K1D, int* bpd, int* Kr, int* bpv) {
@@ -1643,6 +1662,14 @@ int repack_pool(jhq_index* ix, const std::vector<int64_t>& need) {
     return JHQ_OK;
 }
 
+// f() once more with the room of merged batches' workspaces if it does not get
+// its memory.
+template <class F>
+int with_room(jhq_index* ix, F f) {
+    const int rc = f();
+    return drop_merged(ix, rc) ? f() : rc;
+}
+
 // Rotates, encodes and assigns n vectors x (host, dtype) in add_batch chunks
 // (v14/jhq_gpu_index.cu:438-463), inserts them at the end of their lists
 // with ids id_base + i, and grows list blocks as needed.  exact_fit: the
@@ -1782,7 +1809,8 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
             pos += cap;
         }
         if (pos > INT32_MAX) return fail(JHQ_EINVAL, "list pool exceeds int32 slots");
-        JHQ_TRY(grow_pool(ix, pos));  // empty pool: nothing is copied
+        // (empty pool: nothing is copied)
+        JHQ_TRY(with_room(ix, [&] { return grow_pool(ix, pos); }));
         ix->pool_used = pos;
     } else {
         int64_t used = ix->pool_used;
@@ -1805,14 +1833,15 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
             // no room for the moves: re-pack every list instead of growing
             std::vector<int64_t> need(nlist);
             for (int l = 0; l < nlist; l++) need[l] = ix->l_size[l] + add[l + 1];
-            JHQ_TRY(repack_pool(ix, need));
+            JHQ_TRY(with_room(ix, [&] { return repack_pool(ix, need); }));
             moves.clear();
             nstart = ix->l_start;
             ncap = ix->l_cap;
             used = ix->pool_used;
         }
         if (used > INT32_MAX) return fail(JHQ_EINVAL, "list pool exceeds int32 slots");
-        JHQ_TRY(grow_pool(ix, used));  // only an empty pool grows here
+        // (only an empty pool grows here)
+        JHQ_TRY(with_room(ix, [&] { return grow_pool(ix, used); }));
         if (!moves.empty()) {
             DBuf<int4>& dmoves = sc.moves;
             JHQ_TRY(dmoves.upload_keep(moves.data(), moves.size()));
@@ -1868,6 +1897,24 @@ int insert_impl(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_f
     return JHQ_OK;
 }
 
+// An insert and the reservation behind it.  Without memory for its scratch
+// the insert starts over in the room of merged batches' workspaces (nothing has
+// been changed by then).
+int insert_rows(jhq_index* ix, const void* x, int dtype, int64_t n, bool exact_fit) {
+    int rc = insert_impl(ix, x, dtype, n, exact_fit);
+    if (!ix->broken && drop_merged(ix, rc)) {
+        rc = insert_impl(ix, x, dtype, n, exact_fit);
+        if (rc != JHQ_OK && !ix->broken) {
+            const std::string why = g_err;
+            (void)reserve_search(ix);
+            g_err = why;
+        }
+    }
+    JHQ_TRY(rc);
+    ix->added = true;
+    return reserve_search(ix);
+}
+
 int check_insert(jhq_index* ix, const void* x, int64_t n) {
     if (!ix || !x) return fail(JHQ_EINVAL, "null argument");
     if (!ix->trained) return fail(JHQ_ESTATE, "call train() before add()");
@@ -1905,9 +1952,7 @@ int jhq_add_ex(jhq_index* ix, const void* x, int dtype, int64_t n) {
     if (dtype != JHQ_F32 && dtype != JHQ_U8 && dtype != JHQ_I8)
         return fail(JHQ_EINVAL, "unknown dtype");
     if (ix->added || ix->ntotal > 0) return fail(JHQ_ESTATE, "only one add() call is supported");
-    JHQ_TRY(insert_impl(ix, x, dtype, n, true));
-    ix->added = true;
-    return reserve_search(ix);
+    return insert_rows(ix, x, dtype, n, true);
 }
 
 int jhq_append(jhq_index* ix, const float* x, int64_t n) {
@@ -1918,9 +1963,7 @@ int jhq_append_ex(jhq_index* ix, const void* x, int dtype, int64_t n) {
     JHQ_TRY(check_insert(ix, x, n));
     if (dtype != JHQ_F32 && dtype != JHQ_U8 && dtype != JHQ_I8)
         return fail(JHQ_EINVAL, "unknown dtype");
-    JHQ_TRY(insert_impl(ix, x, dtype, n, false));
-    ix->added = true;
-    return reserve_search(ix);
+    return insert_rows(ix, x, dtype, n, false);
 }
 
 int jhq_search(jhq_index* idx, const float* q, int64_t nq, int k, float* dists, int32_t* ids) {
