@@ -210,6 +210,12 @@ int jhq_load(const char* path, jhq_index** out);
  * re-check (mfma_scan_kernel + mfma_recheck_kernel); and the short-list
  * length ck. */
 int jhq_get_plan(const jhq_index* idx, int k, int* scan_kind, int* short_list);
+/* The same for a device call of nq queries as it would run now: the scan, the
+ * queries per batch, the search lanes that get batches, and how many
+ * consecutive batches of a lane share one query product (1: none).  Any
+ * pointer may be NULL. */
+int jhq_get_call_plan(const jhq_index* idx, int64_t nq, int k, int* scan_kind, int* rows, int* lanes,
+                      int* shared);
 
 /* Scan choice (no counterpart in the reference, whose search always runs its
  * byte-LUT scan).  The integer-MFMA pre-scan applies to one-bit digits (K1D =

@@ -95,6 +95,7 @@ _SIGS = {
     "jhq_load": (_I, [ctypes.c_char_p, ctypes.POINTER(_VP)]),
     "jhq_get_params": (_I, [_VP, ctypes.POINTER(_Params)]),
     "jhq_get_plan": (_I, [_VP, _I, ctypes.POINTER(_I), ctypes.POINTER(_I)]),
+    "jhq_get_call_plan": (_I, [_VP, _I64, _I] + [ctypes.POINTER(_I)] * 4),
     "jhq_search_device": (_I, [_VP, _VP, _I64, _I, _VP, _VP, _VP]),
     "jhq_reserve": (_I, [_VP, _I]),
     "jhq_set_scan_kind": (_I, [_VP, _I]),
@@ -157,6 +158,8 @@ def _check(rc):
 
 
 JHQ_F32, JHQ_U8, JHQ_I8 = 0, 1, 2
+_SCANS = ("scan_topck_kernel", "scan_wave_kernel", "scan_dump_kernel", "scan_skew_kernel",
+          "mfma_scan_kernel")
 
 
 def _f32(a, d=None):
@@ -316,9 +319,15 @@ class JHQGpuIndex:
         """(scan kernel name, short-list length ck) a search with this k uses."""
         kind, ck = _I(), _I()
         _check(lib().jhq_get_plan(self._h, int(k), ctypes.byref(kind), ctypes.byref(ck)))
-        names = ("scan_topck_kernel", "scan_wave_kernel", "scan_dump_kernel", "scan_skew_kernel",
-                 "mfma_scan_kernel")
-        return names[kind.value], int(ck.value)
+        return _SCANS[kind.value], int(ck.value)
+
+    def call_plan(self, nq, k):
+        """How search_device runs nq queries: the scan kernel's name, the
+        queries per batch, the lanes that get batches, and the consecutive
+        batches of a lane that share one query product."""
+        v = [_I() for _ in range(4)]
+        _check(lib().jhq_get_call_plan(self._h, int(nq), int(k), *[ctypes.byref(x) for x in v]))
+        return dict(scan=_SCANS[v[0].value], rows=v[1].value, lanes=v[2].value, shared=v[3].value)
 
     def pool(self):
         used, cap = _I64(), _I64()

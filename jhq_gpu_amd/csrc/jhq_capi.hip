@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -868,25 +869,51 @@ int64_t slots_per_query(jhq_index* ix, int P) {
 constexpr int kMergeRows = 512;
 constexpr int64_t kMergeSlots = (int64_t)1 << 26, kMergeScores = (int64_t)1 << 25;
 
+// The k whose plans a reservation covers: the longest short list, the longest
+// that may take the pre-scan, and the shortest.
+std::array<int, 3> planned_ks(const jhq_index* ix) {
+    int kpre = ix->res_k;
+    while (kpre > 1 && ceil_ck(ix->alpha, kpre) > kMfmaMaxCk) kpre--;
+    return {ix->res_k, kpre, 1};
+}
+
 int merged_rows(jhq_index* ix) {
     const int B = ix->batch_size, P = std::min(ix->nprobe, ix->nlist);
-    const int ck = ceil_ck(ix->alpha, ix->res_k), rck = ix->RC * ix->Kr;
+    const int rck = ix->RC * ix->Kr;
     const int64_t perq = slots_per_query(ix, P);
     // (the pre-scan's pair limit holds only where it may be chosen: 4 M x 128, M 16,
     // 64 probes, 2048 queries, B 64: 3260 us in batches of 64, 2535 in merged ones)
     const bool prescan = ix->scan_kind == 2 || (ix->scan_kind == 0 && ix->M >= kMfmaMinM);
-    auto path = [&](int rows, bool* mfma, jhq::ScanShape* sh) {
-        *mfma = prescan && jhq::mfma_scan_ok(ix->M, ix->d, ix->Ds, ix->K1D, ix->bpd, rows, P, ck, rck);
-        return jhq::scan_plan(ix->M, ix->d, P, ck, ix->K1D, rows, ix->num_cu, sh, skew_eligible(ix),
-                              false, rck);
+    struct Path {
+        bool mfma;
+        jhq::ScanShape sh;
+        bool operator==(const Path& o) const {
+            return mfma == o.mfma && sh.wave == o.sh.wave && sh.skew == o.sh.skew &&
+                   sh.dump == o.sh.dump;
+        }
     };
-    bool m0, m1;
-    jhq::ScanShape s0{}, s1{};
-    if (B >= kMergeRows || !path(B, &m0, &s0)) return B;
+    auto path = [&](int k, int rows, Path* p) {
+        const int ck = ceil_ck(ix->alpha, k);
+        p->mfma = prescan && jhq::mfma_scan_ok(ix->M, ix->d, ix->Ds, ix->K1D, ix->bpd, rows, P, ck, rck);
+        p->sh = jhq::ScanShape{};
+        return jhq::scan_plan(ix->M, ix->d, P, ck, ix->K1D, rows, ix->num_cu, &p->sh,
+                              skew_eligible(ix), false, rck);
+    };
+    // Every short list must keep the scan that it has in batches of batch_size
+    // (the longest alone does not tell: where it is past the pre-scan's, 1300 at
+    // M 128 say, it has no pair limit, and the shorter ones would lose the
+    // pre-scan to the merged size).
+    auto same = [&](int rows) {
+        for (int k : planned_ks(ix)) {
+            Path p0, p1;
+            if (!path(k, B, &p0) || !path(k, rows, &p1) || !(p0 == p1)) return false;
+        }
+        return true;
+    };
+    if (B >= kMergeRows) return B;
     for (int rows = kMergeRows / B * B; rows > B; rows -= B)
         if (rows * perq <= kMergeSlots &&
-            static_cast<int64_t>(rows) * (ix->d + ix->nlist) <= kMergeScores && path(rows, &m1, &s1) && m1 == m0 && s1.wave == s0.wave &&
-            s1.skew == s0.skew && s1.dump == s0.dump)
+            static_cast<int64_t>(rows) * (ix->d + ix->nlist) <= kMergeScores && same(rows))
             return rows;
     return B;
 }
@@ -1073,12 +1100,8 @@ bool skew_needed(jhq_index* ix) {
 int reserve_batches(jhq_index* ix) {
     if (ix->skew_stale && skew_needed(ix)) JHQ_TRY(refresh_skew(ix));
     if (rows_wanted(ix) && ix->rows_stale) JHQ_TRY(refresh_rows(ix));
-    // the plans of the longest short list, of the shortest, and of the longest
-    // that may take the pre-scan, for both batch sizes
-    int kpre = ix->res_k;
-    while (kpre > 1 && ceil_ck(ix->alpha, kpre) > kMfmaMaxCk) kpre--;
     BatchPlan bp;
-    for (int k : {ix->res_k, kpre, 1}) {
+    for (int k : planned_ks(ix)) {
         JHQ_TRY(plan_batch(ix, ix->batch_size, k, &bp, kLanes, true));
         if (ix->bcap > ix->batch_size) JHQ_TRY(plan_batch(ix, ix->bcap, k, &bp, kLanes, true));
     }
@@ -1168,6 +1191,25 @@ int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan
     return plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
 }
 
+// The lanes of a pipelined call that get a batch.
+int call_lanes(const jhq_index* ix, int64_t nq, int rows) {
+    return static_cast<int>(std::min<int64_t>(ix->nlanes, (nq + rows - 1) / rows));
+}
+
+// Whether consecutive batches of a device call share their lane's query
+// product: where the selection adds its split sums and every lane has batches
+// enough.
+bool shares_product(const jhq_index* ix, int64_t nq, int rows) {
+    const int d = ix->d, group = qb_share(rows);
+    return group > 1 && ix->dqmat.p && (nq + rows - 1) / rows >= 2 * group * ix->nlanes &&
+           jhq::select_adds_qb(jhq::mfma_qb_plan(rows * group, d + ix->nlist, d), ix->nlist, d);
+}
+
+// A plan's scan as jhq_get_plan and jhq_get_call_plan name it.
+int scan_number(const jhq::ScanShape& sh) {
+    return sh.mfma ? 4 : sh.dump ? 2 : sh.skew ? 3 : sh.wave ? 1 : 0;
+}
+
 // Host arrays over several batches: the batches rotate through the lanes
 // (workspace, pinned staging, stream).  While the other lanes' batches run,
 // the host copies a lane's finished results out and its next queries in.
@@ -1177,8 +1219,7 @@ int search_host_pipelined(jhq_index* ix, const float* q, int64_t nq, int k, cons
     const int Bmax = bp.rows;
     JHQ_TRY(ix->ensure_lanes());
     for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, Bmax, k));
-    // (the lanes that get a batch)
-    const int nl = static_cast<int>(std::min<int64_t>(ix->nlanes, (nq + Bmax - 1) / Bmax));
+    const int nl = call_lanes(ix, nq, Bmax);
     JHQ_HIP(hipEventRecord(ix->lane_ev[0], ix->stream));
     for (int i = 0; i < nl; i++)
         JHQ_HIP(hipStreamWaitEvent(ix->lane[ix->lane_use[i]], ix->lane_ev[0], 0));
@@ -2009,16 +2050,10 @@ int jhq_search_device(jhq_index* ix, const float* d_q, int64_t nq, int k, float*
         ix->done_pending = true;
         return JHQ_OK;
     }
-    // consecutive batches share their lane's query product where the
-    // selection adds its split sums and every lane has batches enough
     const int d = ix->d;
-    const int64_t nb = (nq + Bmax - 1) / Bmax;
     const int group = qb_share(Bmax);
-    const bool share = group > 1 && ix->dqmat.p && nb >= 2 * group * ix->nlanes &&
-                       jhq::select_adds_qb(jhq::mfma_qb_plan(Bmax * group, d + ix->nlist, d),
-                                           ix->nlist, d);
-    // (the lanes that get a batch)
-    const int nl = static_cast<int>(std::min<int64_t>(ix->nlanes, nb));
+    const bool share = shares_product(ix, nq, Bmax);
+    const int nl = call_lanes(ix, nq, Bmax);
     JHQ_HIP(hipEventRecord(ix->lane_ev[0], s));
     for (int i = 0; i < nl; i++)
         JHQ_HIP(hipStreamWaitEvent(ix->lane[ix->lane_use[i]], ix->lane_ev[0], 0));
@@ -2358,8 +2393,23 @@ int jhq_get_plan(const jhq_index* idx, int k, int* scan_kind, int* short_list) {
     if (!jhq::scan_plan(idx->M, idx->d, P, ck, idx->K1D, idx->batch_size, idx->num_cu, &sh,
                         skew_eligible(idx), use_mfma, idx->RC * idx->Kr))
         return fail(JHQ_EINVAL, "no scan plan fits in LDS");
-    if (scan_kind) *scan_kind = sh.mfma ? 4 : sh.dump ? 2 : sh.skew ? 3 : sh.wave ? 1 : 0;
+    if (scan_kind) *scan_kind = scan_number(sh);
     if (short_list) *short_list = ck;
+    return JHQ_OK;
+}
+
+int jhq_get_call_plan(const jhq_index* idx, int64_t nq, int k, int* scan_kind, int* rows, int* lanes,
+                      int* shared) {
+    jhq_index* ix = const_cast<jhq_index*>(idx);  // (a device call's plan changes nothing)
+    JHQ_TRY(check_searchable(ix, nq, k));
+    BatchPlan bp;
+    bool pipe = false;
+    JHQ_TRY(plan_call(ix, std::max<int64_t>(nq, 1), k, false, !ix->timing, &bp, &pipe));
+    if (scan_kind) *scan_kind = scan_number(bp.sh);
+    if (rows) *rows = bp.rows;
+    const int nl = pipe ? call_lanes(ix, nq, bp.rows) : 1;
+    if (lanes) *lanes = nl;
+    if (shared) *shared = pipe && shares_product(ix, nq, bp.rows) ? qb_share(bp.rows) : 1;
     return JHQ_OK;
 }
 

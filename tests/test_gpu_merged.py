@@ -61,3 +61,25 @@ def test_merged_batches_equal_single_ones(built, gpu, kind):
             assert np.array_equal(_bits(od.cpu().numpy()), _bits(want_d[:nq])), nq
     finally:
         ix.set_scan_kind(0)
+
+
+@pytest.mark.parametrize("kind", [0, 2])
+def test_long_short_lists_leave_the_others_their_scan(gpu, kind):
+    """Reserving a k past the pre-scan's short lists changes neither the scan nor
+    the batches of calls with small k (one size serves every reserved k)."""
+    g = np.random.default_rng(8)
+    x = g.standard_normal((4000, 1024)).astype(np.float32)
+    q = g.standard_normal((600, 1024)).astype(np.float32)
+    ix = jg.JHQGpuIndex(1024, jg.Params(M=128, B=8, Br=4, alpha=10.0, nlist=64, nprobe=32,
+                                        ivf_iters=2, batch_size=16, seed=42))
+    ix.train(x[:1000])
+    ix.add(x)
+    ix.set_scan_kind(kind)
+    plan = ix.call_plan(600, 10)
+    assert plan["scan"] == "mfma_scan_kernel" and plan["rows"] == 128
+    want = ix.search(q, 10)
+    ix.reserve(130)
+    assert ix.call_plan(600, 10) == plan
+    assert ix.call_plan(600, 130)["scan"] != "mfma_scan_kernel"
+    got = ix.search(q, 10)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(_bits(got[0]), _bits(want[0]))
