@@ -132,8 +132,8 @@ int jhq_search_ex(jhq_index* idx, const void* q, int dtype, int64_t nq, int k,
  * load() and the setters reserve k_max = 10 at the index's batch_size,
  * nprobe and alpha) and fails with JHQ_ESTATE for a larger k.
  * More than batch_size queries: the call runs in batches of a multiple of
- * batch_size, up to 512 queries as far as the workspace reserved for them
- * stays small; consecutive batches rotate through the
+ * batch_size, up to 512 queries as far as their workspace stays within 640 MB
+ * on each lane in use; consecutive batches rotate through the
  * internal search lanes (a workspace and a stream each; of six created, the
  * ones on hardware queues of their own) forked from `stream`
  * and joined back into it, so the call is stream-ordered on `stream` like a
@@ -145,7 +145,7 @@ int jhq_search_ex(jhq_index* idx, const void* q, int dtype, int64_t nq, int k,
 int jhq_search_device(jhq_index* idx, const float* d_q, int64_t nq, int k,
                       float* d_dists, int32_t* d_ids, void* stream);
 
-/* Preallocates the search workspace (every pipeline lane, pinned staging)
+/* Preallocates the search workspace (every lane in use, pinned staging)
  * for searches with k <= k_max at the current batch_size, nprobe and alpha
  * — the reference's alloc_workspace (v14/jhq_gpu_index.cu:166-206, called at
  * the end of add(), :531) with the ck/k capacities realloc_ck_buffers

@@ -611,26 +611,80 @@ int need(DBuf<T>& b, size_t count, bool grow) {
                 "with this k (after any set_nprobe / set_alpha) before a device search");
 }
 
-int ensure_workspace(jhq_index* ix, Workspace& w, int ck, int k, int P, int max_segments,
-                     bool grow) {
-    const size_t B = static_cast<size_t>(ix->bcap);
-    if (grow) ix->ws_rows = std::max(ix->ws_rows, ix->bcap);
-    JHQ_TRY(need(w.wq, B * ix->d, grow));
-    JHQ_TRY(need(w.wqrot, B * ix->d, grow));
-    JHQ_TRY(need(w.wscores, B * ix->nlist, grow));
-    JHQ_TRY(need(w.wprobes, B * P, grow));
-    JHQ_TRY(need(w.wgofs, B * (P + 1), grow));
-    JHQ_TRY(need(w.wqtot, B, grow));
-    JHQ_TRY(need(w.wpartial, static_cast<size_t>(max_segments) * ck, grow));
-    JHQ_TRY(need(w.wpslot, static_cast<size_t>(max_segments) * ck, grow));
-    JHQ_TRY(need(w.wtopck, B * ck, grow));
-    JHQ_TRY(need(w.wout_d, B * k, grow));
-    JHQ_TRY(need(w.wout_i, B * k, grow));
-    if (ix->dqmat.p) {
-        // split sums of the largest product
-        const size_t pf = jhq::mfma_qb_space(ix->bcap * qb_share(ix->bcap), ix->d + ix->nlist, ix->d);
-        if (pf) JHQ_TRY(need(w.wqpart, pf, grow));
+// Candidate slots a query can have at most: the padded sizes of the P largest
+// lists (cached per P; inserts reset the cache).
+int64_t slots_per_query(jhq_index* ix, int P) {
+    if (ix->dump_P != P) {
+        std::vector<int32_t> sz(ix->l_size);
+        std::partial_sort(sz.begin(), sz.begin() + P, sz.end(), std::greater<int32_t>());
+        int64_t per_q = 0;
+        for (int i = 0; i < P; i++)
+            per_q += (sz[i] + jhq::kGroup - 1) / jhq::kGroup * jhq::kGroup;
+        ix->dump_P = P;
+        ix->dump_perq = std::max<int64_t>(per_q, 1);
     }
+    return ix->dump_perq;
+}
+
+// Elements of a lane's search buffers for batches of `rows` queries under a
+// plan (P probes, short list ck, scan shape sh).
+struct WsNeed {
+    size_t q = 0, scores = 0, probes = 0, gofs = 0, qtot = 0, partial = 0, topck = 0, out = 0;
+    size_t qpart = 0;  // split sums of the largest product
+    size_t dump = 0, mfma = 0;
+    // grown with an eighth to spare: appends lengthen the lists a little at a
+    // time, and each reallocation here is one per lane
+    size_t dump_grown() const { return dump + dump / 8; }
+    size_t bytes() const {
+        return 4 * (2 * q + scores + probes + gofs + qtot + partial + qpart) +
+               8 * (partial + topck + out + dump_grown()) + mfma;
+    }
+    void cover(const WsNeed& o) {
+        for (auto f : {&WsNeed::q, &WsNeed::scores, &WsNeed::probes, &WsNeed::gofs, &WsNeed::qtot,
+                       &WsNeed::partial, &WsNeed::topck, &WsNeed::out, &WsNeed::qpart, &WsNeed::dump,
+                       &WsNeed::mfma})
+            this->*f = std::max(this->*f, o.*f);
+    }
+};
+
+WsNeed ws_need(jhq_index* ix, int rows, int ck, int k, int P, const jhq::ScanShape& sh) {
+    const size_t B = static_cast<size_t>(rows);
+    WsNeed n;
+    n.q = B * ix->d;
+    n.scores = B * ix->nlist;
+    n.probes = B * P;
+    n.gofs = B * (P + 1);
+    n.qtot = B;
+    n.partial = static_cast<size_t>(sh.max_segments) * ck;
+    n.topck = B * ck;
+    n.out = B * k;
+    if (ix->dqmat.p) n.qpart = jhq::mfma_qb_space(rows * qb_share(rows), ix->d + ix->nlist, ix->d);
+    if (sh.dump || sh.mfma) {
+        // keys (dump scan) or biased integer distances (MFMA pre-scan: u32 slots
+        // and one tile minimum per 16 after them)
+        const size_t slots = B * slots_per_query(ix, P);
+        n.dump = sh.mfma ? (slots + slots / 16 + 40) / 2 : slots;
+    }
+    if (sh.mfma) n.mfma = jhq::mfma_scan_bytes(rows, P, ix->M, ix->num_cu);
+    return n;
+}
+
+int ensure_workspace(jhq_index* ix, Workspace& w, const WsNeed& n, bool grow) {
+    if (grow) ix->ws_rows = std::max(ix->ws_rows, ix->bcap);
+    JHQ_TRY(need(w.wq, n.q, grow));
+    JHQ_TRY(need(w.wqrot, n.q, grow));
+    JHQ_TRY(need(w.wscores, n.scores, grow));
+    JHQ_TRY(need(w.wprobes, n.probes, grow));
+    JHQ_TRY(need(w.wgofs, n.gofs, grow));
+    JHQ_TRY(need(w.wqtot, n.qtot, grow));
+    JHQ_TRY(need(w.wpartial, n.partial, grow));
+    JHQ_TRY(need(w.wpslot, n.partial, grow));
+    JHQ_TRY(need(w.wtopck, n.topck, grow));
+    JHQ_TRY(need(w.wout_d, n.out, grow));
+    JHQ_TRY(need(w.wout_i, n.out, grow));
+    if (n.qpart) JHQ_TRY(need(w.wqpart, n.qpart, grow));
+    if (n.dump && !w.wdump.has(n.dump)) JHQ_TRY(need(w.wdump, grow ? n.dump_grown() : n.dump, grow));
+    if (n.mfma) JHQ_TRY(need(w.wmfma, n.mfma, grow));
     return JHQ_OK;
 }
 
@@ -840,21 +894,6 @@ struct BatchPlan {
     jhq::ScanShape sh;
 };
 
-// Candidate slots a query can have at most: the padded sizes of the P largest
-// lists (cached per P; inserts reset the cache).
-int64_t slots_per_query(jhq_index* ix, int P) {
-    if (ix->dump_P != P) {
-        std::vector<int32_t> sz(ix->l_size);
-        std::partial_sort(sz.begin(), sz.begin() + P, sz.end(), std::greater<int32_t>());
-        int64_t per_q = 0;
-        for (int i = 0; i < P; i++)
-            per_q += (sz[i] + jhq::kGroup - 1) / jhq::kGroup * jhq::kGroup;
-        ix->dump_P = P;
-        ix->dump_perq = std::max<int64_t>(per_q, 1);
-    }
-    return ix->dump_perq;
-}
-
 // Queries per batch of a call with more than batch_size of them: as many whole
 // batch_size's as fit in kMergeRows.  A batch is a chain of 4 to 6 launches
 // whose time hardly depends on its queries while they are few, and larger ones
@@ -863,11 +902,11 @@ int64_t slots_per_query(jhq_index* ix, int P) {
 // x 100 int8, 320 queries, B 32: 584 us, 315, 258, 202, 202; 300 K x 384, k 100,
 // 4000 queries, B 128: 2243, 2212, 1866, 1725, 1735; 262 K x 1024, 4096 queries,
 // B 64: 2200, 1968, 1844 (then the pair limit); 20 K x 96, 37 queries, B 16: 150
-// us, in one batch 88.  Not past the pre-scan's pair limit, the LDS plan,
-// kMergeSlots candidate slots of dump buffer (512 MB of keys) or kMergeScores
-// score floats (128 MB) per lane.
+// us, in one batch 88.  Not past the pre-scan's pair limit, the LDS plan or
+// kMergeBytes of workspace on each lane (four of them hold one with HIP's
+// default queues: 2.5 GB of the card's 288).
 constexpr int kMergeRows = 512;
-constexpr int64_t kMergeSlots = (int64_t)1 << 26, kMergeScores = (int64_t)1 << 25;
+constexpr size_t kMergeBytes = (size_t)640 << 20;
 
 // The k whose plans a reservation covers: the longest short list, the longest
 // that may take the pre-scan, and the shortest.
@@ -880,7 +919,6 @@ std::array<int, 3> planned_ks(const jhq_index* ix) {
 int merged_rows(jhq_index* ix) {
     const int B = ix->batch_size, P = std::min(ix->nprobe, ix->nlist);
     const int rck = ix->RC * ix->Kr;
-    const int64_t perq = slots_per_query(ix, P);
     // (the pre-scan's pair limit holds only where it may be chosen: 4 M x 128, M 16,
     // 64 probes, 2048 queries, B 64: 3260 us in batches of 64, 2535 in merged ones)
     const bool prescan = ix->scan_kind == 2 || (ix->scan_kind == 0 && ix->M >= kMfmaMinM);
@@ -903,25 +941,38 @@ int merged_rows(jhq_index* ix) {
     // (the longest alone does not tell: where it is past the pre-scan's, 1300 at
     // M 128 say, it has no pair limit, and the shorter ones would lose the
     // pre-scan to the merged size).
-    auto same = [&](int rows) {
+    auto fits = [&](int rows) {
+        WsNeed n;
         for (int k : planned_ks(ix)) {
             Path p0, p1;
             if (!path(k, B, &p0) || !path(k, rows, &p1) || !(p0 == p1)) return false;
+            const int ck = ceil_ck(ix->alpha, k);
+            n.cover(ws_need(ix, rows, ck, k, P, p1.sh));
+            if (p1.mfma && jhq::scan_plan(ix->M, ix->d, P, ck, ix->K1D, rows, ix->num_cu, &p1.sh, false,
+                                          true, rck))
+                n.cover(ws_need(ix, rows, ck, k, P, p1.sh));
         }
-        return true;
+        return n.bytes() <= kMergeBytes;
     };
     if (B >= kMergeRows) return B;
     for (int rows = kMergeRows / B * B; rows > B; rows -= B)
-        if (rows * perq <= kMergeSlots &&
-            static_cast<int64_t>(rows) * (ix->d + ix->nlist) <= kMergeScores && same(rows))
-            return rows;
+        if (fits(rows)) return rows;
     return B;
 }
 
-// The plan of a search batch and the workspaces it needs on nws lanes.
+// f(l) for each lane that a call's batches run on: lane 0 alone, or (pipe) those
+// in use.
+template <class F>
+int each_lane(const jhq_index* ix, bool pipe, F f) {
+    if (!pipe) return f(0);
+    for (int i = 0; i < ix->nlanes; i++) JHQ_TRY(f(ix->lane_use[i]));
+    return JHQ_OK;
+}
+
+// The plan of a search batch and the workspaces it needs on its lanes.
 // grow = false (device searches): nothing is allocated or refreshed, and a
 // shape beyond the reservation fails with JHQ_ESTATE.
-int plan_batch(jhq_index* ix, int Bq, int k, BatchPlan* bp, int nws, bool grow) {
+int plan_batch(jhq_index* ix, int Bq, int k, BatchPlan* bp, bool pipe, bool grow) {
     bp->Bq = bp->rows = Bq;
     bp->ck = ceil_ck(ix->alpha, k);
     bp->P = std::min(ix->nprobe, ix->nlist);
@@ -940,24 +991,9 @@ int plan_batch(jhq_index* ix, int Bq, int k, BatchPlan* bp, int nws, bool grow) 
         if (!grow) return fail(JHQ_ESTATE, "the row-major code copy is out of date");
         JHQ_TRY(refresh_rows(ix));
     }
-    for (int i = 0; i < nws; i++)
-        JHQ_TRY(ensure_workspace(ix, ix->ws[i], bp->ck, k, bp->P, bp->sh.max_segments, grow));
-    if (bp->sh.dump || bp->sh.mfma) {
-        // keys (dump scan) or biased integer distances (MFMA pre-scan)
-        // (the pre-scan: u32 slots and one tile minimum per 16 after them)
-        // (grown with an eighth to spare: appends lengthen the lists a little
-        // at a time, and each reallocation here is one per lane)
-        const size_t slots = static_cast<size_t>(ix->bcap) * slots_per_query(ix, bp->P);
-        const size_t words = bp->sh.mfma ? (slots + slots / 16 + 40) / 2 : slots;
-        for (int i = 0; i < nws; i++)
-            if (!ix->ws[i].wdump.has(words))
-                JHQ_TRY(need(ix->ws[i].wdump, grow ? words + words / 8 : words, grow));
-        if (bp->sh.mfma)
-            for (int i = 0; i < nws; i++)
-                JHQ_TRY(need(ix->ws[i].wmfma,
-                             jhq::mfma_scan_bytes(ix->bcap, bp->P, ix->M, ix->num_cu), grow));
-    }
-    return JHQ_OK;
+    if (grow && pipe) JHQ_TRY(ix->ensure_lanes());
+    const WsNeed n = ws_need(ix, ix->bcap, bp->ck, k, bp->P, bp->sh);
+    return each_lane(ix, pipe, [&](int l) { return ensure_workspace(ix, ix->ws[l], n, grow); });
 }
 
 // One batch of Bq queries at d_q (device) through the whole pipeline
@@ -1102,12 +1138,11 @@ int reserve_batches(jhq_index* ix) {
     if (rows_wanted(ix) && ix->rows_stale) JHQ_TRY(refresh_rows(ix));
     BatchPlan bp;
     for (int k : planned_ks(ix)) {
-        JHQ_TRY(plan_batch(ix, ix->batch_size, k, &bp, kLanes, true));
-        if (ix->bcap > ix->batch_size) JHQ_TRY(plan_batch(ix, ix->bcap, k, &bp, kLanes, true));
+        JHQ_TRY(plan_batch(ix, ix->batch_size, k, &bp, true, true));
+        if (ix->bcap > ix->batch_size) JHQ_TRY(plan_batch(ix, ix->bcap, k, &bp, true, true));
     }
-    JHQ_TRY(ix->ensure_lanes());
-    for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, ix->bcap, ix->res_k));
-    return JHQ_OK;
+    return each_lane(ix, true,
+                     [&](int l) { return ensure_host_staging(ix, l, ix->bcap, ix->res_k); });
 }
 
 // After a failed allocation: merged batches are not worth failing for (their
@@ -1176,7 +1211,7 @@ int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan
         rows = static_cast<int>(std::min<int64_t>(rows, (nq + parts - 1) / parts));
     }
     if (merge && nq > ix->batch_size && rows > ix->batch_size) {
-        const int rc = plan_batch(ix, ix->bcap, k, bp, nq > rows ? kLanes : 1, grow);
+        const int rc = plan_batch(ix, ix->bcap, k, bp, nq > rows, grow);
         if (rc == JHQ_OK) {
             bp->rows = rows;
             *pipe = nq > rows;
@@ -1185,10 +1220,10 @@ int plan_call(jhq_index* ix, int64_t nq, int k, bool grow, bool merge, BatchPlan
         if (grow && drop_merged(ix, rc)) (void)reserve_batches(ix);
     }
     *pipe = merge && nq > ix->batch_size;
-    const int rc = plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
+    const int rc = plan_batch(ix, ix->batch_size, k, bp, *pipe, grow);
     if (!grow || !drop_merged(ix, rc)) return rc;
     (void)reserve_batches(ix);
-    return plan_batch(ix, ix->batch_size, k, bp, *pipe ? kLanes : 1, grow);
+    return plan_batch(ix, ix->batch_size, k, bp, *pipe, grow);
 }
 
 // The lanes of a pipelined call that get a batch.
@@ -1217,8 +1252,7 @@ int search_host_pipelined(jhq_index* ix, const float* q, int64_t nq, int k, cons
                           float* dists, int32_t* ids) {
     const int d = ix->d;
     const int Bmax = bp.rows;
-    JHQ_TRY(ix->ensure_lanes());
-    for (int l = 0; l < kLanes; l++) JHQ_TRY(ensure_host_staging(ix, l, Bmax, k));
+    JHQ_TRY(each_lane(ix, true, [&](int l) { return ensure_host_staging(ix, l, Bmax, k); }));
     const int nl = call_lanes(ix, nq, Bmax);
     JHQ_HIP(hipEventRecord(ix->lane_ev[0], ix->stream));
     for (int i = 0; i < nl; i++)

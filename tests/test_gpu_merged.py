@@ -83,3 +83,26 @@ def test_long_short_lists_leave_the_others_their_scan(gpu, kind):
     assert ix.call_plan(600, 130)["scan"] != "mfma_scan_kernel"
     got = ix.search(q, 10)
     assert np.array_equal(got[1], want[1]) and np.array_equal(_bits(got[0]), _bits(want[0]))
+
+
+def test_workspaces_stay_within_their_bound(gpu):
+    """The workspaces of merged batches: at most 640 MB on each lane that a call
+    uses (one list of 131072 and k 100: 577 MB of distances for 512 queries)."""
+    import torch
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    g = np.random.default_rng(9)
+    x = g.standard_normal((131072, 64)).astype(np.float32)
+    ix = jg.JHQGpuIndex(64, jg.Params(M=16, B=8, Br=4, alpha=4.0, nlist=1, nprobe=1, ivf_iters=1,
+                                      batch_size=32, seed=42))
+    ix.train(x[:2000])
+    ix.add(x)
+    before = used()
+    ix.reserve(100)
+    plan = ix.call_plan(1 << 16, 100)
+    assert plan["rows"] == 512 and plan["scan"] == "scan_dump_kernel"
+    assert used() - before <= plan["lanes"] * (640 << 20)
