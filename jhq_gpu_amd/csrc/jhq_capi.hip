@@ -752,7 +752,7 @@ int mfma_measure_cost(jhq_index* ix, int B, int P, double* cost, double* cand) {
     JHQ_HIP(jhq::decode_rows(dsamp.p, S, ix->dcodes_t.p, ix->M, ix->Ds, ix->K1D, ix->bpd,
                              ix->dc1d.p, rows.p, st));
     JHQ_HIP(jhq::mfma_nt_score(rows.p, d, ix->dcent.p, d, S, nlist, d, ix->dnorms.p, scores.p,
-                               nlist, st));
+                               nlist, S, st));
     JHQ_HIP(jhq::select_probes(scores.p, S, nlist, P, ix->dldesc.p, probes.p, gofs.p, qtot.p, st));
     std::vector<int32_t> hp(static_cast<size_t>(S) * P);
     JHQ_HIP(hipMemcpyAsync(hp.data(), probes.p, hp.size() * sizeof(int32_t),
@@ -1038,10 +1038,12 @@ int run_batch(jhq_index* ix, Workspace& w, const float* d_q, int Bq, int k, cons
                                  w.wqrot.p, d, w.wscores.p, ix->nlist, ix->dnorms.p, w.wqpart.p,
                                  w.wqpart.n, s, !sel_qb));
     } else {
-        // d not a multiple of 64: the 16-row kernels
-        JHQ_HIP(jhq::mfma_nt_store(d_q, d, ix->dP.p, d, Bq, d, d, w.wqrot.p, d, s));
+        // d not a multiple of 64: the 16-row kernels; merged batches sum in the
+        // order of batches of batch_size
+        const int split = std::min(Bq, ix->batch_size);
+        JHQ_HIP(jhq::mfma_nt_store(d_q, d, ix->dP.p, d, Bq, d, d, w.wqrot.p, d, split, s));
         JHQ_HIP(jhq::mfma_nt_score(w.wqrot.p, d, ix->dcent.p, d, Bq, ix->nlist, d, ix->dnorms.p,
-                                   w.wscores.p, ix->nlist, s));
+                                   w.wscores.p, ix->nlist, split, s));
     }
     if (ix->timing) JHQ_HIP(hipEventRecord(ix->ev[1], s));
     const jhq::PrescanSel* psp = bp.sh.mfma ? &ps : nullptr;

@@ -67,10 +67,14 @@ hipError_t mfma_qb(const QbPlan& p, const float* A, int64_t lda, const float* Bm
                    int nb, int N, int K, int nrot, float* C1, int64_t ld1, float* C2, int64_t ld2,
                    const float* norms, float* part, size_t part_floats, hipStream_t s,
                    bool reduce = true);
+// The same products for any K, 16 rows x 16 columns a workgroup.  K is split over
+// its waves as split_rows rows need it to fill the chip: the split, and with it
+// the order of a row's sums, does not depend on nb.
 hipError_t mfma_nt_store(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb, int N,
-                         int K, float* C, int64_t ldc, hipStream_t s);
+                         int K, float* C, int64_t ldc, int split_rows, hipStream_t s);
 hipError_t mfma_nt_score(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb, int N,
-                         int K, const float* norms, float* C, int64_t ldc, hipStream_t s);
+                         int K, const float* norms, float* C, int64_t ldc, int split_rows,
+                         hipStream_t s);
 // uint8 (dtype 1) / int8 (dtype 2) elements to float32.
 hipError_t convert_to_f32(const void* src, int dtype, int64_t n, float* dst, hipStream_t s);
 hipError_t fill_u64(unsigned long long* p, int64_t n, unsigned long long v, hipStream_t s);

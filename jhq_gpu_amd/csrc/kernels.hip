@@ -655,9 +655,9 @@ hipError_t mfma_qb(const QbPlan& p, const float* A, int64_t lda, const float* Bm
 template <int EPI>
 static hipError_t launch_mfma(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb,
                               int N, int K, float* C, int64_t ldc, const float* norms,
-                              hipStream_t s) {
+                              int split_rows, hipStream_t s) {
     if (nb <= 0 || N <= 0) return hipSuccess;
-    const int64_t tiles = (int64_t)((N + 15) / 16) * ((nb + 15) / 16);
+    const int64_t tiles = (int64_t)((N + 15) / 16) * ((split_rows + 15) / 16);
     if ((nb + 15) / 16 > 65535) return hipErrorInvalidValue;
     int S = 1;
     while (S < 8 && tiles * S < 2048 && K / (S * 2) >= 64) S *= 2;
@@ -682,13 +682,14 @@ static hipError_t launch_mfma(const float* A, int64_t lda, const float* Bm, int6
 }
 
 hipError_t mfma_nt_store(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb, int N,
-                         int K, float* C, int64_t ldc, hipStream_t s) {
-    return launch_mfma<EPI_STORE>(A, lda, Bm, ldb, nb, N, K, C, ldc, nullptr, s);
+                         int K, float* C, int64_t ldc, int split_rows, hipStream_t s) {
+    return launch_mfma<EPI_STORE>(A, lda, Bm, ldb, nb, N, K, C, ldc, nullptr, split_rows, s);
 }
 
 hipError_t mfma_nt_score(const float* A, int64_t lda, const float* Bm, int64_t ldb, int nb, int N,
-                         int K, const float* norms, float* C, int64_t ldc, hipStream_t s) {
-    return launch_mfma<EPI_SCORE>(A, lda, Bm, ldb, nb, N, K, C, ldc, norms, s);
+                         int K, const float* norms, float* C, int64_t ldc, int split_rows,
+                         hipStream_t s) {
+    return launch_mfma<EPI_SCORE>(A, lda, Bm, ldb, nb, N, K, C, ldc, norms, split_rows, s);
 }
 
 // Stored vectors decoded from their primary codes (rotated space, each

@@ -1,7 +1,8 @@
 """Search calls with more queries than batch_size run in merged batches of up
 to 512 queries: the ids and distances of every call are, bit for bit, those of
-one call per batch_size queries (host and device, each scan kind, sizes around
-the merged batch, the lanes and a ragged last batch)."""
+calls of batch_size queries (host and device, each scan kind, sizes around the
+merged batch, the lanes and a ragged last batch, and shapes whose products are
+split over K by the number of rows)."""
 import numpy as np
 import pytest
 
@@ -18,6 +19,11 @@ SHAPES = {
     "flat": (96, 12, 8, 1, 1, 7, 4.0, 1),
     "long_lists": (128, 32, 4, 16, 16, 100, 4.0, 100),
     "batch_over_512": (64, 16, 4, 16, 4, 600, 4.0, 10),
+    # d not a multiple of 64: the rows would choose the split of the scores (2 at
+    # 64 rows, 1 at 512; only near ties of the probes show it) and of the
+    # rotation (8 and 2; every distance shows it)
+    "split_scores": (200, 50, 4, 2048, 8, 64, 4.0, 10),
+    "split_rotation": (520, 65, 4, 16, 4, 64, 4.0, 10),
 }
 
 
