@@ -177,9 +177,9 @@ static_assert(kLanes >= 1, "at least one lane");
 #endif
 constexpr int kQbShare = JHQ_QB_SHARE;
 static_assert(kQbShare >= 1, "at least one batch per product");
-// Batches of more than 128 queries keep their own (262 K x 1024 in batches of
-// 128: 2190 us a call on products of their own, 2079 on shared ones; 256: no
-// difference).
+// Batches of more than 128 queries keep their own: 262 K x 1024, 16 probes, 16
+// batches of 256: 1410 us on products of their own, 1420 on shared ones, and no
+// gain at 2 to 12 batches.
 constexpr int qb_share(int batch) { return batch <= 128 ? kQbShare : 1; }
 
 // Per-batch search buffers (v14/search.cuh:24-46).  The index keeps one set
@@ -1234,8 +1234,12 @@ int call_lanes(const jhq_index* ix, int64_t nq, int rows) {
 }
 
 // Whether consecutive batches of a device call share their lane's query
-// product: where the selection adds its split sums and every lane has batches
-// enough.
+// product: where the selection adds its split sums and every lane gets two
+// pairs or more.  262 K vectors on four lanes, us a call on products of their
+// own and on shared ones: 1024 dimensions, 32 probes, 4 batches of 128: 271
+// and 312 (half of the lanes idle), 12: 692 and 723, 16: 904 and 890, 32: 1736
+// and 1700; 64 probes, 48 batches of 64: 1800 and 1767; 512 dimensions, 16
+// batches of 128: 619 and 604, 24: 894 and 871.
 bool shares_product(const jhq_index* ix, int64_t nq, int rows) {
     const int d = ix->d, group = qb_share(rows);
     return group > 1 && ix->dqmat.p && (nq + rows - 1) / rows >= 2 * group * ix->nlanes &&

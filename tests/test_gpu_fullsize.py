@@ -142,14 +142,16 @@ def test_cfg2_full_stagewise(gpu, nprobe):
 
 @pytest.mark.parametrize("nprobe", [16, 64])
 def test_cfg2_full_device_search_lanes(gpu, nprobe):
-    """Seven batches through the pipelined device search (the search lanes; three
-    pairs that each share one query product, then one batch alone) equal the
-    debug search of the same queries, batch by batch on one stream."""
+    """A pipelined device search (the search lanes; merged batches of 256 queries
+    at 16 probes, batches of 64 at 64) equals the debug search of the same
+    queries, batch by batch on one stream."""
     import torch
     g, o, hb, hq, cb, L = _cfg2(gpu)
     g.set_nprobe(nprobe)
     try:
         g.reserve(10)
+        plan = g.call_plan(NQ_DEVICE, 10)
+        assert plan["rows"] == 4096 // nprobe and plan["lanes"] > 1
         want = g.search_debug(hq, 10)
         qt = torch.from_numpy(hq).to(gpu)
         od = torch.full((NQ_DEVICE, 10), -1.0, dtype=torch.float32, device=gpu)

@@ -69,6 +69,39 @@ def test_merged_batches_equal_single_ones(built, gpu, kind):
         ix.set_scan_kind(0)
 
 
+@pytest.mark.parametrize("d,M,nprobe", [(1024, 128, 32), (1024, 128, 64), (512, 64, 64)])
+def test_batches_sharing_a_query_product(gpu, d, M, nprobe):
+    """Many batches of at most 128 queries: a lane takes two at a time with one
+    query product (4 split sums a query at d 1024, 2 at 512), the last pair
+    ragged, or its last batch alone."""
+    import torch
+    g = np.random.default_rng(6)
+    x = g.standard_normal((3000, d)).astype(np.float32)
+    ix = jg.JHQGpuIndex(d, jg.Params(M=M, B=8, Br=4, alpha=4.0, nlist=96, nprobe=nprobe,
+                                     ivf_iters=2, batch_size=64, seed=42))
+    ix.train(x[:1000])
+    ix.add(x)
+    ix.set_scan_kind(2)
+    rows = ix.call_plan(1 << 16, 10)["rows"]
+    assert rows == 4096 // nprobe
+    many = 4 * ix.call_plan(1 << 16, 10)["lanes"]
+    q = g.standard_normal(((many + 1) * rows + rows // 2, d)).astype(np.float32)
+    parts = [ix.search(q[i:i + 64], 10) for i in range(0, len(q), 64)]
+    want_d = np.concatenate([p[0] for p in parts])
+    want_i = np.concatenate([p[1] for p in parts])
+    qt = torch.from_numpy(q).to(gpu)
+    for nq in (len(q), len(q) - rows, many * rows):
+        plan = ix.call_plan(nq, 10)
+        assert plan["shared"] == 2 and plan["lanes"] > 1, (nq, plan)
+        od = torch.full((nq, 10), -1.0, device=gpu)
+        oi = torch.full((nq, 10), -2, dtype=torch.int32, device=gpu)
+        for _ in range(2):
+            ix.search_device(qt[:nq], 10, od, oi, stream=torch.cuda.current_stream())
+            assert np.array_equal(oi.cpu().numpy(), want_i[:nq]), nq
+            assert np.array_equal(_bits(od.cpu().numpy()), _bits(want_d[:nq])), nq
+    assert ix.call_plan((many - 1) * rows, 10)["shared"] == 1
+
+
 @pytest.mark.parametrize("kind", [0, 2])
 def test_long_short_lists_leave_the_others_their_scan(gpu, kind):
     """Reserving a k past the pre-scan's short lists changes neither the scan nor

@@ -153,14 +153,15 @@ def test_mfma_after_appends(gpu):
 
 
 def test_mfma_device_search_pipelined(gpu):
-    """Many batches of a device search (the search lanes, one workspace each;
-    consecutive batch pairs of a lane share one query product, the last pair
-    ragged) return what the host search returns."""
+    """Many merged batches of a device search (the search lanes, one workspace
+    each, the last batch ragged) return what the host search returns."""
     import torch
     g, o, q, k = _build(CASES[IDS.index("m32_a4")])
-    batch = CASES[IDS.index("m32_a4")][-1]
     g.reserve(k)
-    qq = np.ascontiguousarray(np.tile(q, (1 + 5 * batch // q.shape[0], 1))[:5 * batch + 3])
+    nq = 5 * g.call_plan(1 << 16, k)["rows"] + 3
+    plan = g.call_plan(nq, k)
+    assert plan["lanes"] > 1 and plan["scan"] == "mfma_scan_kernel"
+    qq = np.ascontiguousarray(np.tile(q, (1 + nq // q.shape[0], 1))[:nq])
     d1, i1 = g.search(qq, k)
     qt = torch.from_numpy(qq).to(gpu)
     od = torch.full((qq.shape[0], k), -1.0, dtype=torch.float32, device=gpu)

@@ -211,17 +211,19 @@ def test_search_device_matches_host(gpu, case):
 
 @pytest.mark.parametrize("name", ["ds8_k1d2", "m64_ds4_ck100", "k100_ck400", "d1024_m128"])
 def test_search_device_pipelined_batches(gpu, name):
-    """A device search over many batches (the search lanes, each a workspace and a stream,
-    joined into the caller's stream; consecutive batch pairs of a lane share one
-    query product where the probe selection adds its split sums, as at d = 1024) returns what
-    one call per batch and the host search return, including a ragged last
-    batch (the second of the last pair)."""
+    """A device search over many merged batches (the search lanes, each a workspace
+    and a stream, joined into the caller's stream) returns what one call per
+    batch_size queries and the host search return, including a ragged last
+    batch."""
     import torch
     case = CASES[IDS.index(name)]
     g, o, base, q, k = _build(case)
     batch = case[-1]
     g.reserve(k)  # device searches run in the reserved workspace only
-    qq = np.ascontiguousarray(np.tile(q, (1 + 5 * batch // q.shape[0], 1))[:5 * batch + 3])
+    nq = 5 * g.call_plan(1 << 16, k)["rows"] + 3
+    plan = g.call_plan(nq, k)
+    assert nq > 5 * batch and plan["lanes"] > 1 and nq // plan["rows"] == 5
+    qq = np.ascontiguousarray(np.tile(q, (1 + nq // q.shape[0], 1))[:nq])
     d1, i1 = g.search(qq, k)
     qt = torch.from_numpy(qq).to(gpu)
     od = torch.full((qq.shape[0], k), -1.0, dtype=torch.float32, device=gpu)
