@@ -1234,15 +1234,22 @@ int call_lanes(const jhq_index* ix, int64_t nq, int rows) {
 }
 
 // Whether consecutive batches of a device call share their lane's query
-// product: where the selection adds its split sums and every lane gets two
-// pairs or more.  262 K vectors on four lanes, us a call on products of their
-// own and on shared ones: 1024 dimensions, 32 probes, 4 batches of 128: 271
-// and 312 (half of the lanes idle), 12: 692 and 723, 16: 904 and 890, 32: 1736
-// and 1700; 64 probes, 48 batches of 64: 1800 and 1767; 512 dimensions, 16
-// batches of 128: 619 and 604, 24: 894 and 871.
+// product: where the selection adds its split sums and no lane gets more batches
+// in groups than one by one.  131 K to 262 K vectors on four lanes, us a call on
+// products of their own and on shared ones: 1024 dimensions, 32 probes, batches
+// of 128: 4 of them 227 and 277 (half of the lanes idle), 5: 331 and 300, 6: 344
+// and 329, 8: 400 and 409, 10: 545 and 643, 12: 582 and 665, 14: 700 and 706,
+// 18: 871 and 967, 24: 1108 and 1118, 60: 2683 and 2723; 64 probes, batches of
+// 64: 4: 186 and 246, 5: 271 and 267, 7: 305 and 291, 10: 413 and 474, 14: 542
+// and 536, 18: 670 and 722, 24: 831 and 815; 512 dimensions, 32 probes, batches
+// of 128: 5: 246 and 227, 8: 294 and 291, 12: 415 and 440, 14: 499 and 477, 20:
+// 657 and 669, 24: 774 and 747, 60: 1846 and 1812.
 bool shares_product(const jhq_index* ix, int64_t nq, int rows) {
     const int d = ix->d, group = qb_share(rows);
-    return group > 1 && ix->dqmat.p && (nq + rows - 1) / rows >= 2 * group * ix->nlanes &&
+    if (group < 2 || !ix->dqmat.p) return false;
+    const int64_t nb = (nq + rows - 1) / rows, nl = call_lanes(ix, nq, rows);
+    const int64_t groups = (nb + group - 1) / group;
+    return group * ((groups + nl - 1) / nl) <= (nb + nl - 1) / nl &&
            jhq::select_adds_qb(jhq::mfma_qb_plan(rows * group, d + ix->nlist, d), ix->nlist, d);
 }
 

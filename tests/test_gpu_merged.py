@@ -71,9 +71,9 @@ def test_merged_batches_equal_single_ones(built, gpu, kind):
 
 @pytest.mark.parametrize("d,M,nprobe", [(1024, 128, 32), (1024, 128, 64), (512, 64, 64)])
 def test_batches_sharing_a_query_product(gpu, d, M, nprobe):
-    """Many batches of at most 128 queries: a lane takes two at a time with one
-    query product (4 split sums a query at d 1024, 2 at 512), the last pair
-    ragged, or its last batch alone."""
+    """Batches of at most 128 queries: a lane takes two at a time with one query
+    product (4 split sums a query at d 1024, 2 at 512), the last pair ragged, or
+    its last batch alone."""
     import torch
     g = np.random.default_rng(6)
     x = g.standard_normal((3000, d)).astype(np.float32)
@@ -84,13 +84,15 @@ def test_batches_sharing_a_query_product(gpu, d, M, nprobe):
     ix.set_scan_kind(2)
     rows = ix.call_plan(1 << 16, 10)["rows"]
     assert rows == 4096 // nprobe
-    many = 4 * ix.call_plan(1 << 16, 10)["lanes"]
-    q = g.standard_normal(((many + 1) * rows + rows // 2, d)).astype(np.float32)
+    L = ix.call_plan(1 << 16, 10)["lanes"]
+    assert L > 1
+    q = g.standard_normal((4 * L * rows, d)).astype(np.float32)
     parts = [ix.search(q[i:i + 64], 10) for i in range(0, len(q), 64)]
     want_d = np.concatenate([p[0] for p in parts])
     want_i = np.concatenate([p[1] for p in parts])
     qt = torch.from_numpy(q).to(gpu)
-    for nq in (len(q), len(q) - rows, many * rows):
+    # in batches: whole pairs, a ragged last one, a last batch alone
+    for nq in (len(q), len(q) - rows // 2, len(q) - rows, L * rows + 1):
         plan = ix.call_plan(nq, 10)
         assert plan["shared"] == 2 and plan["lanes"] > 1, (nq, plan)
         od = torch.full((nq, 10), -1.0, device=gpu)
@@ -99,7 +101,10 @@ def test_batches_sharing_a_query_product(gpu, d, M, nprobe):
             ix.search_device(qt[:nq], 10, od, oi, stream=torch.cuda.current_stream())
             assert np.array_equal(oi.cpu().numpy(), want_i[:nq]), nq
             assert np.array_equal(_bits(od.cpu().numpy()), _bits(want_d[:nq])), nq
-    assert ix.call_plan((many - 1) * rows, 10)["shared"] == 1
+    # pairs where they lengthen no lane: 2 or 4 batches on the fullest one, not 1
+    # or 3
+    for nb in range(1, 4 * L + 1):
+        assert ix.call_plan(nb * rows, 10)["shared"] == (1 if (nb + L - 1) // L % 2 else 2), nb
 
 
 @pytest.mark.parametrize("kind", [0, 2])
