@@ -7,6 +7,7 @@
 #include "../../include/jhq.h"
 #include "host_train.h"
 #include "kernels.h"
+#include "lanes.h"
 
 #include <hip/hip_runtime.h>
 
@@ -386,28 +387,27 @@ struct jhq_index {
     // sat idle half of a search).  A one-wave kernel of fixed length runs on
     // the lanes taken so far and on the next lane at once: if they finish
     // within 1.5 times one kernel's time, the next lane has a queue of its
-    // own and is taken.  Any failure leaves every lane in use.
+    // own and is taken (pick_lanes).  Any failure leaves every lane in use.
     void calibrate_lanes() {
         nlanes = kLanes;
         for (int l = 0; l < kLanes; l++) lane_use[l] = l;
         if (kLanes < 2) return;
         float* buf = nullptr;
         hipEvent_t e0 = nullptr, e1[kLanes] = {};
-        int use[kLanes], n = 1;
-        use[0] = 0;
+        int use[kLanes];
         bool ok = hipMalloc(reinterpret_cast<void**>(&buf), kLanes * sizeof(float)) == hipSuccess &&
                   hipEventCreate(&e0) == hipSuccess;
         for (int l = 0; ok && l < kLanes; l++) ok = hipEventCreate(&e1[l]) == hipSuccess;
         // the span from the first lane's start to the last lane's end
-        auto span = [&](const int* ls, int m, float* ms) {
+        auto span = [&](const int* ls, int m, bool brief, float* ms) {
             // about 270 us (200000 steps took 2.7 ms, and the 20 or so runs of a new
             // index's calibration 28 of its add()'s 31 ms)
-            constexpr int kIters = 20000;
+            const int iters = brief ? 16 : 20000;
             if (hipEventRecord(e0, lane[ls[0]]) != hipSuccess) return false;
             for (int i = 1; i < m; i++)
                 if (hipStreamWaitEvent(lane[ls[i]], e0, 0) != hipSuccess) return false;
             for (int i = 0; i < m; i++)
-                if (jhq::lane_probe(buf + ls[i], kIters, lane[ls[i]]) != hipSuccess ||
+                if (jhq::lane_probe(buf + ls[i], iters, lane[ls[i]]) != hipSuccess ||
                     hipEventRecord(e1[i], lane[ls[i]]) != hipSuccess)
                     return false;
             *ms = 0.f;
@@ -420,14 +420,8 @@ struct jhq_index {
             }
             return true;
         };
-        float t1 = 0.f, t = 0.f;
-        ok = ok && span(use, 1, &t1) && span(use, 1, &t1) && t1 > 0.f;  // the first run loads the kernel
-        for (int j = 1; ok && j < kLanes; j++) {
-            use[n] = j;
-            ok = span(use, n + 1, &t);
-            if (ok && t < 1.5f * t1) n++;
-        }
-        if (ok && n >= 1) {
+        const int n = ok ? jhq::pick_lanes(kLanes, use, span) : 0;
+        if (n >= 1) {
             nlanes = n;
             for (int i = 0; i < n; i++) lane_use[i] = use[i];
         }
