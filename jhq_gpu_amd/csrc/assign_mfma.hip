@@ -186,8 +186,10 @@ __device__ __forceinline__ void push_candidate(const CollectIO& io, int64_t slot
 }
 
 // The 16 RT rows of a wave in TOP2: lane (r, g) keeps rows 16 i + 4 g + j over
-// its columns (r of every group of 16).  A NaN score makes s2 = s1 (the row
-// is re-checked): v_med3 of a NaN is the smaller of the others.
+// its columns (r of every group of 16).  A NaN score is never the best, as in
+// the fixed order, where its key is above every number's; s becomes b then
+// (v_med3 of a NaN is the smaller of the others), so that the row is
+// re-checked unless a score smaller by more than the bound follows.
 template <int RT>
 struct Top2State {
     float b[RT][4], s[RT][4];

@@ -63,169 +63,169 @@ gemm_chain_kernel(const float* __restrict__ A, int64_t lda, const float* __restr
     if (ROWS) n = min(n, (int64_t)*ndev);
     // (without ROWS the grid covers the tiles: one pass)
     for (int64_t item = blockIdx.x;; item += gridDim.x) {
-    const int64_t slot = item >> 3;
-    const int64_t row0 = ((item & 7) + 8 * (slot / ncol)) * BT;
-    const int col0 = (int)(slot % ncol) * BT;
-    if (row0 >= n) {
-        if (!ROWS || slot / ncol * 8 * BT >= n) return;
-        continue;
-    }
-    if (ROWS) __syncthreads();  // the previous tile's reads are done
+        const int64_t slot = item >> 3;
+        const int64_t row0 = ((item & 7) + 8 * (slot / ncol)) * BT;
+        const int col0 = (int)(slot % ncol) * BT;
+        if (row0 >= n) {
+            if (!ROWS || slot / ncol * 8 * BT >= n) return;
+            continue;
+        }
+        if (ROWS) __syncthreads();  // the previous tile's reads are done
 
-    // thread t stages 4 k from 4 (t % 8) of rows t / 8 + 32 i
-    const int lk = 4 * (tid & 7), lr = tid >> 3;
-    const float* ap[L];
-    const float* bp[L];
-#pragma unroll
-    for (int i = 0; i < L; i++) {
-        const int64_t row = min(row0 + lr + 32 * i, n - 1);
-        ap[i] = A + (ROWS ? (int64_t)rowidx[row] : row) * lda;
-        bp[i] = Bm + (int64_t)min(col0 + lr + 32 * i, m - 1) * ldb;
-    }
-    float4 ra[L], rb[L];
-    // a whole k step: plain loads, no test behind them, so that they stay in
-    // flight over the step before (a zero selected for k past d made the
-    // compiler wait for each load: 102 TFLOP/s at 65536 x 1024 x 1024)
-    auto load = [&](int k0) {
+        // thread t stages 4 k from 4 (t % 8) of rows t / 8 + 32 i
+        const int lk = 4 * (tid & 7), lr = tid >> 3;
+        const float* ap[L];
+        const float* bp[L];
 #pragma unroll
         for (int i = 0; i < L; i++) {
-            const float* pa = ap[i] + k0 + lk;
-            const float* pb = bp[i] + k0 + lk;
-            if (VEC) {
-                ra[i] = *(const float4*)pa;
-                rb[i] = *(const float4*)pb;
-            } else {
-                ra[i] = make_float4(pa[0], pa[1], pa[2], pa[3]);
-                rb[i] = make_float4(pb[0], pb[1], pb[2], pb[3]);
+            const int64_t row = min(row0 + lr + 32 * i, n - 1);
+            ap[i] = A + (ROWS ? (int64_t)rowidx[row] : row) * lda;
+            bp[i] = Bm + (int64_t)min(col0 + lr + 32 * i, m - 1) * ldb;
+        }
+        float4 ra[L], rb[L];
+        // a whole k step: plain loads, no test behind them, so that they stay in
+        // flight over the step before (a zero selected for k past d made the
+        // compiler wait for each load: 102 TFLOP/s at 65536 x 1024 x 1024)
+        auto load = [&](int k0) {
+#pragma unroll
+            for (int i = 0; i < L; i++) {
+                const float* pa = ap[i] + k0 + lk;
+                const float* pb = bp[i] + k0 + lk;
+                if (VEC) {
+                    ra[i] = *(const float4*)pa;
+                    rb[i] = *(const float4*)pb;
+                } else {
+                    ra[i] = make_float4(pa[0], pa[1], pa[2], pa[3]);
+                    rb[i] = make_float4(pb[0], pb[1], pb[2], pb[3]);
+                }
             }
-        }
-    };
-    // the last step of d % 32 k
-    auto load_tail = [&](int k0) {
-        auto at = [&](const float* p, int k) { return k < d ? p[k] : 0.0f; };
-        const int k = k0 + lk;
+        };
+        // the last step of d % 32 k
+        auto load_tail = [&](int k0) {
+            auto at = [&](const float* p, int k) { return k < d ? p[k] : 0.0f; };
+            const int k = k0 + lk;
 #pragma unroll
-        for (int i = 0; i < L; i++) {
-            ra[i] = make_float4(at(ap[i], k), at(ap[i], k + 1), at(ap[i], k + 2), at(ap[i], k + 3));
-            rb[i] = make_float4(at(bp[i], k), at(bp[i], k + 1), at(bp[i], k + 2), at(bp[i], k + 3));
-        }
-    };
-    // k of a block of 8: even ones at 0..3, odd ones at 4..7
-    const int st = (lk & ~7) + (lk & 4) / 2;
-    auto store = [&]() {
+            for (int i = 0; i < L; i++) {
+                ra[i] = make_float4(at(ap[i], k), at(ap[i], k + 1), at(ap[i], k + 2), at(ap[i], k + 3));
+                rb[i] = make_float4(at(bp[i], k), at(bp[i], k + 1), at(bp[i], k + 2), at(bp[i], k + 3));
+            }
+        };
+        // k of a block of 8: even ones at 0..3, odd ones at 4..7
+        const int st = (lk & ~7) + (lk & 4) / 2;
+        auto store = [&]() {
 #pragma unroll
-        for (int i = 0; i < L; i++) {
-            // the pairs are put together here, not (with a wait) behind the loads
-            asm volatile("" : "+v"(ra[i].x), "+v"(ra[i].y), "+v"(ra[i].z), "+v"(ra[i].w));
-            asm volatile("" : "+v"(rb[i].x), "+v"(rb[i].y), "+v"(rb[i].z), "+v"(rb[i].w));
-            *(float2*)&As[lr + 32 * i][st] = make_float2(ra[i].x, ra[i].z);
-            *(float2*)&As[lr + 32 * i][st + 4] = make_float2(ra[i].y, ra[i].w);
-            *(float2*)&Bs[lr + 32 * i][st] = make_float2(rb[i].x, rb[i].z);
-            *(float2*)&Bs[lr + 32 * i][st + 4] = make_float2(rb[i].y, rb[i].w);
-        }
-    };
+            for (int i = 0; i < L; i++) {
+                // the pairs are put together here, not (with a wait) behind the loads
+                asm volatile("" : "+v"(ra[i].x), "+v"(ra[i].y), "+v"(ra[i].z), "+v"(ra[i].w));
+                asm volatile("" : "+v"(rb[i].x), "+v"(rb[i].y), "+v"(rb[i].z), "+v"(rb[i].w));
+                *(float2*)&As[lr + 32 * i][st] = make_float2(ra[i].x, ra[i].z);
+                *(float2*)&As[lr + 32 * i][st + 4] = make_float2(ra[i].y, ra[i].w);
+                *(float2*)&Bs[lr + 32 * i][st] = make_float2(rb[i].x, rb[i].z);
+                *(float2*)&Bs[lr + 32 * i][st + 4] = make_float2(rb[i].y, rb[i].w);
+            }
+        };
 
-    v16f_c acc[T][T];
+        v16f_c acc[T][T];
 #pragma unroll
-    for (int i = 0; i < T; i++)
-#pragma unroll
-        for (int j = 0; j < T; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    auto step = [&]() {
-#pragma unroll
-        for (int kk = 0; kk < kChainBK; kk += 8) {
-            v4f_c a[T], b[T];
-#pragma unroll
-            for (int i = 0; i < T; i++)
-                a[i] = *(const v4f_c*)&As[32 * (wr * T + i) + l32][kk + 4 * h];
+        for (int i = 0; i < T; i++)
 #pragma unroll
             for (int j = 0; j < T; j++)
-                b[j] = *(const v4f_c*)&Bs[32 * (wc * T + j) + l32][kk + 4 * h];
 #pragma unroll
-            for (int s = 0; s < 4; s++)
+                for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
+
+        auto step = [&]() {
+#pragma unroll
+            for (int kk = 0; kk < kChainBK; kk += 8) {
+                v4f_c a[T], b[T];
 #pragma unroll
                 for (int i = 0; i < T; i++)
+                    a[i] = *(const v4f_c*)&As[32 * (wr * T + i) + l32][kk + 4 * h];
 #pragma unroll
-                    for (int j = 0; j < T; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], b[j][s],
-                                                                         acc[i][j], 0, 0, 0);
-        }
-    };
-    const int dw = d / kChainBK * kChainBK;  // whole steps
-    if (dw > 0) load(0);
-    for (int k0 = 0; k0 < dw; k0 += kChainBK) {
-        store();
-        __syncthreads();
-        // (the last pass loads its own step again)
-        load(min(k0 + kChainBK, dw - kChainBK));
-        __builtin_amdgcn_sched_barrier(0);  // the loads are issued before the MFMAs
-        step();
-        __syncthreads();
-    }
-    if (dw < d) {
-        load_tail(dw);
-        store();
-        __syncthreads();
-        step();
-    }
-
-    // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
-    auto row_of = [&](int i, int r) {
-        return row0 + 32 * (wr * T + i) + 8 * (r / 4) + 4 * h + r % 4;
-    };
+                for (int j = 0; j < T; j++)
+                    b[j] = *(const v4f_c*)&Bs[32 * (wc * T + j) + l32][kk + 4 * h];
 #pragma unroll
-    for (int i = 0; i < T; i++) {
-        if constexpr (EPI == CHAIN_STORE) {
+                for (int s = 0; s < 4; s++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int64_t row = row_of(i, r);
-                if (row < n) {
+                    for (int i = 0; i < T; i++)
 #pragma unroll
-                    for (int j = 0; j < T; j++) {
-                        const int col = col0 + 32 * (wc * T + j) + l32;
-                        if (col < m) C[row * ldc + col] = acc[i][j][r];
-                    }
-                }
+                        for (int j = 0; j < T; j++)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][s], b[j][s],
+                                                                             acc[i][j], 0, 0, 0);
             }
-        } else {
-            unsigned long long best[16];
+        };
+        const int dw = d / kChainBK * kChainBK;  // whole steps
+        if (dw > 0) load(0);
+        for (int k0 = 0; k0 < dw; k0 += kChainBK) {
+            store();
+            __syncthreads();
+            // (the last pass loads its own step again)
+            load(min(k0 + kChainBK, dw - kChainBK));
+            __builtin_amdgcn_sched_barrier(0);  // the loads are issued before the MFMAs
+            step();
+            __syncthreads();
+        }
+        if (dw < d) {
+            load_tail(dw);
+            store();
+            __syncthreads();
+            step();
+        }
+
+        // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32
+        auto row_of = [&](int i, int r) {
+            return row0 + 32 * (wr * T + i) + 8 * (r / 4) + 4 * h + r % 4;
+        };
 #pragma unroll
-            for (int r = 0; r < 16; r++) best[r] = ~0ull;
-#pragma unroll
-            for (int j = 0; j < T; j++) {
-                const int col = col0 + 32 * (wc * T + j) + l32;
-                if (col >= m) continue;
-                const float nc = norms[col];
+        for (int i = 0; i < T; i++) {
+            if constexpr (EPI == CHAIN_STORE) {
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
-                    const float sc = fmaf(-2.0f, acc[i][j][r], nc);
-                    const unsigned long long key =
-                        ((unsigned long long)chain_ord(sc) << 32) | (uint32_t)col;
-                    best[r] = key < best[r] ? key : best[r];
-                }
-            }
-            // minimum over the 32 columns of a lane half: each round a lane
-            // keeps half of its rows and hands the others to its partner
-            // (16 exchanges instead of 80)
+                    const int64_t row = row_of(i, r);
+                    if (row < n) {
 #pragma unroll
-            for (int c = 8; c >= 1; c >>= 1) {
-                const bool up = (l32 & (2 * c)) != 0;
-#pragma unroll
-                for (int r = 0; r < c; r++) {
-                    const unsigned long long keep = up ? best[r + c] : best[r];
-                    const unsigned long long o = __shfl_xor(up ? best[r] : best[r + c], 2 * c);
-                    best[r] = o < keep ? o : keep;
+                        for (int j = 0; j < T; j++) {
+                            const int col = col0 + 32 * (wc * T + j) + l32;
+                            if (col < m) C[row * ldc + col] = acc[i][j][r];
+                        }
+                    }
                 }
+            } else {
+                unsigned long long best[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) best[r] = ~0ull;
+#pragma unroll
+                for (int j = 0; j < T; j++) {
+                    const int col = col0 + 32 * (wc * T + j) + l32;
+                    if (col >= m) continue;
+                    const float nc = norms[col];
+#pragma unroll
+                    for (int r = 0; r < 16; r++) {
+                        const float sc = fmaf(-2.0f, acc[i][j][r], nc);
+                        const unsigned long long key =
+                            ((unsigned long long)chain_ord(sc) << 32) | (uint32_t)col;
+                        best[r] = key < best[r] ? key : best[r];
+                    }
+                }
+                // minimum over the 32 columns of a lane half: each round a lane
+                // keeps half of its rows and hands the others to its partner
+                // (16 exchanges instead of 80)
+#pragma unroll
+                for (int c = 8; c >= 1; c >>= 1) {
+                    const bool up = (l32 & (2 * c)) != 0;
+#pragma unroll
+                    for (int r = 0; r < c; r++) {
+                        const unsigned long long keep = up ? best[r + c] : best[r];
+                        const unsigned long long o = __shfl_xor(up ? best[r] : best[r + c], 2 * c);
+                        best[r] = o < keep ? o : keep;
+                    }
+                }
+                const unsigned long long o = __shfl_xor(best[0], 1);
+                const unsigned long long key = o < best[0] ? o : best[0];
+                const int64_t row = row_of(i, l32 >> 1);
+                if (!(l32 & 1) && row < n && key != ~0ull) atomicMin(&keys[row], key);
             }
-            const unsigned long long o = __shfl_xor(best[0], 1);
-            const unsigned long long key = o < best[0] ? o : best[0];
-            const int64_t row = row_of(i, l32 >> 1);
-            if (!(l32 & 1) && row < n && key != ~0ull) atomicMin(&keys[row], key);
         }
-    }
-    if (!ROWS) return;
+        if (!ROWS) return;
     }
 }
 
@@ -255,7 +255,9 @@ static hipError_t launch_chain(const float* A, int64_t lda, const float* Bm, int
 // workgroups: 2000 x 768 has 96 of the large (a third of the chip, 41 us of MFMAs
 // in each) and 384 of the small (34 us measured); from 512 on the large ones win
 // by their fewer LDS reads per MFMA (64 x 64: 16 bytes per lane for 4, 128 x 128
-// for 8)
+// for 8).  The small ones down to one row (a kernel with 1 to 8 rows per thread on
+// the vector ALU took, and these take, us: 1 x 1024 24.5 and 23.0, 64 x 1024 25.6
+// and 23.8, 512 x 1024 108 and 24, 1 x 128 5.3 and 4.7, 64 x 128 5.7 and 5.1)
 static bool chain_small(int64_t n, int m) {
     return ((n + 127) / 128) * ((m + 127) / 128) < 512;
 }

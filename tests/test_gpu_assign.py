@@ -70,3 +70,22 @@ def test_assign_non_finite(gpu, d):
     want = _assign(gpu, jg.k_assign_noalloc, y, cent, norms)
     ok = np.isfinite(y).all(1)
     assert np.array_equal(got[ok], want[ok]) and np.array_equal(got[~ok], want[~ok])
+
+
+@pytest.mark.parametrize("d", [32, 132, 320])
+@pytest.mark.parametrize("first", [True, False], ids=["before", "behind"])
+def test_assign_nan_lists(gpu, d, first):
+    """Lists with a NaN among finite ones, and finite rows: the bound stays finite,
+    so the rows are accepted or re-checked by their own scores.  The NaN lists,
+    before or behind the others, are no row's."""
+    rng = np.random.default_rng(d)
+    cent = rng.standard_normal((150, d)).astype(np.float32)
+    nan = np.arange(0, 20, 3) if first else np.arange(130, 150, 3)
+    cent[nan, rng.integers(0, d, len(nan))] = np.nan
+    y = rng.standard_normal((500, d)).astype(np.float32)
+    y[:100] = 0.5 * (cent[50] + cent[rng.integers(20, 130, 100)])  # near ties
+    norms = po.cent_norms(cent)
+    got = _assign(gpu, jg.k_assign, y, cent, norms)
+    finite = np.setdiff1d(np.arange(150), nan)
+    assert np.array_equal(got, finite[po.assign(y, cent[finite], norms[finite])])
+    assert np.array_equal(got, _assign(gpu, jg.k_assign_noalloc, y, cent, norms))

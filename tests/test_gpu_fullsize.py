@@ -1,5 +1,5 @@
 """GPU parity at the benchmarked operating point, full size: config 2
-(BASELINE.json configs[1]) with N = 1,000,000, D = 1024, nlist = 4096, M = 128,
+with N = 1,000,000, D = 1024, nlist = 4096, M = 128,
 batch 64, alpha 10 (ck = 100), nprobe 16 and 64.
 
 The index is built by the GPU (train on the first 100,000 vectors, then one

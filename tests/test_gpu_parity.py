@@ -1,6 +1,6 @@
 """GPU parity: the HIP product against the CPU oracle on identical seeded inputs.
 
-Bar (BASELINE.json north_star): codebooks, rotation, codes and list layout are
+Bar: codebooks, rotation, codes and list layout are
 bit-exact.  Search is checked stage-wise: the query rotation and centroid
 scores run on fp32 MFMA, so the oracle is fed the GPU's rotated queries (checked
 against float64) and its probe lists (checked against the oracle's own

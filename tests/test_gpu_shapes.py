@@ -1,4 +1,4 @@
-"""GPU parity at the shapes the benchmark runs (BASELINE.json configs), smaller N.
+"""GPU parity at the shapes the benchmark runs, smaller N.
 
 Every shape here has one-bit digits, so it can run the integer-MFMA pre-scan
 with exact re-check (forced with scan kind 2) or the byte-LUT scans (scan kind
