@@ -1,9 +1,9 @@
 #!/usr/bin/env python3
 """bench.py — JHQ IVF search throughput on one MI355X.
 
-Default run (the driver's `python bench.py --gpus 1 --steps K --warmup W`):
+Default run (`python bench.py --gpus 1 --steps K --warmup W`):
 
-* Headline, BASELINE.json configs[1] ("config 2"): N=1,000,000 base and
+* Headline ("config 2"): N=1,000,000 base and
   10,000 query vectors, D=1024 fp32, drawn from a seeded 10,000-component
   Gaussian mixture (per-component N(0, I) mean, diagonal std log-uniform in
   [0.1, 1], uniform weights) and L2-normalised.  IVF nlist=4096 trained on the
@@ -21,7 +21,7 @@ Default run (the driver's `python bench.py --gpus 1 --steps K --warmup W`):
   0.001 of the best recall.  `value` is that point's queries/s over exactly
   --steps timed steps; the host-to-host rate of the reference's protocol
   (PCIe copies included) is reported beside it.
-* HBM-streaming leg, configs[2] ("config 3"): 100M x 128 uint8, nlist 65,536,
+* HBM-streaming leg ("config 3"): 100M x 128 uint8, nlist 65,536,
   nprobe 64, M=16, batch 64 (1.6 GB of codes, streamed from HBM), under
   `hbm_streaming_leg` with its own roofline, counters and build check.
 
@@ -60,8 +60,8 @@ def parse():
                          "configs 3-5)")
     ap.add_argument("--warmup", type=int, default=0, help="warmup steps (default: 1)")
     ap.add_argument("--config", type=int, default=None, choices=(1, 2, 3, 4, 5),
-                    help="BASELINE.json workload alone: 2 (the metric's config), 1 (flat "
-                         "100K x 1024, one query per batch), 3 (100M uint8 D=128), 4 (100M "
+                    help="one workload alone: 2 (the metric's config), 1 (flat "
+                         "100K x 1024, batch_size 1), 3 (100M uint8 D=128), 4 (100M "
                          "int8 D=100), 5 (streaming add + search, D=768).  Default: config 2, "
                          "then config 3 as the HBM-streaming leg of the same JSON line")
     ap.add_argument("--no-hbm-leg", action="store_true",
@@ -77,7 +77,7 @@ def parse():
     ap.add_argument("--profile-batches", type=int, default=0,
                     help="profiling mode: build the index, run this many search batches at the "
                          "first --nprobe/--alpha plus one 256 MiB device copy (the counter "
-                         "calibration kernel), print per-step times and exit")
+                         "calibration kernel) and exit")
     ap.add_argument("--trace-steps", type=int, default=0,
                     help="kernel-trace mode: build the index, then run one warmup and this many "
                          "timed device-search calls over the whole query set at the first "
@@ -183,12 +183,12 @@ def main():
 
 
 FLOAT_CFGS = {
-    # flat JHQ, one query at a time
+    # flat JHQ, queries of a call in batches of batch_size 1 or merged ones
     1: dict(name="cfg1", N=100_000, NQ=1_000, NCOMP=1_000, D=1024, M=128, NLIST=1, NPROBE="1",
             ALPHA="4", BATCH=1, seed=0x4A48510001,
             workload="cfg1 flat JHQ N=100K D=1024 fp32, nlist=1, M=128 B=8 Br=4, alpha=%g, "
-                     "k=10, one query per batch, queries resident in HBM"),
-    # BASELINE.json configs[1]: the metric's config
+                     "k=10, batch_size 1, queries resident in HBM"),
+    # the metric's config
     2: dict(name="cfg2", N=1_000_000, NQ=10_000, NCOMP=10_000, D=1024, M=128, NLIST=4096,
             NPROBE="16,32,64", ALPHA="4,10", BATCH=64, seed=0x4A48510002,
             workload="cfg2 IVF-JHQ N=1M D=1024 fp32, nlist=4096, M=128 B=8 Br=4, alpha=%g, "
@@ -365,7 +365,8 @@ def bench_float(args, cf):
         "config": {
             "workload": cf["workload"] % alpha,
             "N": N, "nq": NQ, "nlist": NLIST, "nprobe": npb, "alpha": alpha, "k": K,
-            "batch": BATCH, "recall_at_10": round(rec, 4),
+            "batch": BATCH, "queries_per_timed_batch": roof["queries_per_batch"],
+            "recall_at_10": round(rec, 4),
             "recall_gate_0.95_met": gate_met,
             "recall_at_10_ceiling_all_refined": round(ceiling, 4),
             "recall_at_10_reference_definition": round(rec_ref, 4),
@@ -576,7 +577,9 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
 
     Time base: one batch's share of the timed pipelined run, ev_ms_per_step /
     batches per step (HIP events on the caller's stream bracket the timed steps;
-    the engine forks its lanes from that stream and joins them back into it).
+    the engine forks its lanes from that stream and joins them back into it).  A
+    batch is what the timed call runs as one (a multiple of batch_size: call_plan);
+    kernel_alone has the batches of batch_size that the per-step timing runs.
 
     Bytes and ops are what the dominant step's kernels must move and compute:
     * byte-LUT scans (scan_skew / scan_wave / scan_dump): every probed code is
@@ -599,23 +602,26 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
     sizes = np.diff(L["offsets"]).astype(np.int64)
     pad = (sizes + 15) // 16
     nq = hq.shape[0]
-    nb = (nq + batch - 1) // batch
     M, D = ix.params.M, hq.shape[1]
     kernel, ck = ix.scan_plan(k)
     bpv = ix.dims()["bpv"]
     probes = dbg["probes"]
-    codes_per_query = float(sizes[probes].sum()) * M / nb       # per batch, counted per query
-    refine = float(nq) * ck * (bpv + 4 + 4) / nb
-    t_batch = ev_ms_per_step * 1e3 / nb                          # us per batch, pipelined
     mfma = kernel == "mfma_scan_kernel"
     fused = mfma and ck <= 128
     alone_us = step_us["scan_topck"] + (0.0 if fused else step_us["refine_topk"])
-    parts = {"refine": refine}
-    ops = 0.0
-    if mfma:
+
+    def per_batch(rows_of):
+        """Bytes by part, int8 ops, tile row reads and codes counted per query, of
+        a batch of rows_of queries (the mean over the batches of a call)."""
+        nb = (nq + rows_of - 1) // rows_of
+        codes = float(sizes[probes].sum()) * M / nb
+        parts = {"refine": float(nq) * ck * (bpv + 4 + 4) / nb}
+        if not mfma:
+            parts["codes_per_query"] = codes
+            return nb, parts, 0.0, 0, codes
         distinct = rows = tiles = 0
         for b in range(nb):
-            lists, cnt = np.unique(probes[b * batch:(b + 1) * batch], return_counts=True)
+            lists, cnt = np.unique(probes[b * rows_of:(b + 1) * rows_of], return_counts=True)
             distinct += int(sizes[lists].sum()) * M
             rows += int((((cnt + 15) // 16) * sizes[lists]).sum()) * M
             tiles += int((((cnt + 15) // 16) * pad[lists]).sum())
@@ -624,16 +630,19 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
         dump_r = float((qt * 4 + np.minimum(qt, ck) * 16 * 4).sum())
         parts.update(codes_distinct_lists=distinct / nb, dump_write=dump_w / nb,
                      dump_read_min=dump_r / nb)
-        ops = tiles / nb * 16.0 * 16.0 * D * 2 * 2
-    else:
-        parts["codes_per_query"] = codes_per_query
+        return nb, parts, tiles / nb * 16.0 * 16.0 * D * 2 * 2, rows / nb, codes
+
+    run_rows = ix.call_plan(nq, k)["rows"]                       # queries of a timed batch
+    nb, parts, ops, tile_rows, codes_per_query = per_batch(run_rows)
+    t_batch = ev_ms_per_step * 1e3 / nb                          # us per batch, pipelined
+    _, alone_parts, _, _, alone_codes = per_batch(batch)
     step_bytes = sum(parts.values())
     gbs = step_bytes / (t_batch * 1e-6) / 1e9
     tops = ops / (t_batch * 1e-6) / 1e12
     f_hbm, f_mfma = gbs / HBM_PEAK_GBS, tops / INT8_PEAK_TOPS
     bound = "mfma" if f_mfma > f_hbm else "hbm"
     traffic, traffic_note, limiter = None, "no counter run at this operating point", None
-    counters = None
+    counters = traffic_rows = None
     pdir = os.path.join(ROOT, "profiles")
     for fn in sorted(os.listdir(pdir)) if (use_profiles and os.path.isdir(pdir)) else []:
         if not fn.endswith("_traffic.json"):
@@ -642,11 +651,13 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
             tj = json.load(f)
         if (tj.get("kernel") == kernel and tj.get("nprobe") == nprobe
                 and float(tj.get("alpha")) == float(alpha)
-                and tj.get("workload", "").startswith(workload)):
+                and tj.get("workload", "").startswith(workload)
+                and (traffic is None or tj["queries_per_launch"] == run_rows)):
             traffic = int(tj["traffic_bytes_per_launch"])
             traffic_note = ("HBM bytes per launch of the step's kernels from %s (FETCH_SIZE x %.2f "
                             "+ WRITE_SIZE x %.2f, factors from a copy kernel of known size)"
                             % (tj["source"], tj["fetch_scale"], tj["write_scale"]))
+            traffic_rows = tj["queries_per_launch"]
             limiter = tj.get("limiter")
             counters = tj.get("counters")
     names = {"scan_dump_kernel": "scan_dump_kernel + select_query_kernel",
@@ -662,29 +673,32 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
         "frac": round(max(f_hbm, f_mfma), 4),
         "traffic": traffic,
         "time_base": "us per batch in the timed pipelined run: HIP events on the caller's "
-                     "stream around the timed steps / batches of batch_size per step (bytes and "
-                     "ops counted per such batch; the engine merges batches, which read "
-                     "fewer of their shared lists than this counts)",
+                     "stream around the timed steps / batches per step; bytes and ops "
+                     "counted per such batch",
+        "queries_per_batch": run_rows,
         "us_per_batch_pipelined": round(t_batch, 2),
         "algorithmic_bytes_per_batch": int(step_bytes),
         "bytes_breakdown": {k2: int(v) for k2, v in parts.items()},
         "hbm": {"achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "frac": round(f_hbm, 4)},
         "traffic_note": traffic_note,
-        "traffic_rate_over_step_gbs": (None if traffic is None
+        "traffic_queries_per_launch": traffic_rows,
+        "traffic_rate_over_step_gbs": (None if traffic is None or traffic_rows != run_rows
                                        else round(traffic / (t_batch * 1e-6) / 1e9, 1)),
         "limiter": limiter,
         "counters": counters,
         "kernel_alone": {
             "us_per_launch": round(alone_us, 2),
-            "note": "the step's kernels on one stream (HIP events in a separate timing pass); "
-                    "in the pipelined run other lanes' kernels run beside them",
-            "frac_hbm": round(step_bytes / (alone_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
+            "queries_per_launch": batch,
+            "note": "the step's kernels on one stream (HIP events in a separate timing pass, in "
+                    "batches of batch_size); in the pipelined run other lanes' kernels run "
+                    "beside them",
+            "frac_hbm": round(sum(alone_parts.values()) / (alone_us * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
         },
     }
     if mfma:
         out["int8_mfma"] = {"ops_per_batch": int(ops), "achieved_tops": round(tops, 2),
                             "peak_tops": INT8_PEAK_TOPS, "frac": round(f_mfma, 4)}
-        out["tile_row_reads_per_batch"] = int(rows / nb)
+        out["tile_row_reads_per_batch"] = int(tile_rows)
         out["effective_per_query_codes"] = {
             "bytes_per_batch": int(codes_per_query),
             "gbs_over_step": round(codes_per_query / (t_batch * 1e-6) / 1e9, 1),
@@ -695,8 +709,9 @@ def step_roofline(ix, hq, k, batch, step_us, ev_ms_per_step, workload, nprobe, a
     else:
         out["scan_kernel_alone"] = {
             "us_per_launch": round(step_us["scan_topck"], 2),
-            "codes_bytes_per_launch": int(codes_per_query),
-            "frac_hbm": round(codes_per_query / (step_us["scan_topck"] * 1e-6) / 1e9
+            "queries_per_launch": batch,
+            "codes_bytes_per_launch": int(alone_codes),
+            "frac_hbm": round(alone_codes / (step_us["scan_topck"] * 1e-6) / 1e9
                               / HBM_PEAK_GBS, 4),
         }
     return out
@@ -811,7 +826,8 @@ def bench_bytes(args, cf):
                         f"B=8 Br=4, alpha={alpha:g}, k=10, batch={BATCH}, queries resident "
                         "in HBM",
             "N": N, "nq": NQ, "nlist": NLIST, "nprobe": npb, "alpha": alpha, "k": K,
-            "batch": BATCH, "n_train": n_train,
+            "batch": BATCH, "queries_per_timed_batch": roof["queries_per_batch"],
+            "n_train": n_train,
             "recall_at_10": round(rec, 4), "recall_at_10_tie_aware": round(rec_tie, 4),
             "recall_at_10_reference_definition": round(rec_ref, 4),
             "build_s": {"train": round(t_train, 2), "add": round(t_add, 2)},
@@ -955,7 +971,8 @@ def bench_streaming(args):
                         f"{BATCH}-query searches, D=768, nlist={NLIST}, M=96 per-subspace "
                         f"residual codebooks, alpha={alpha:g}, k=100",
             "N_final": upto, "nq": NQ, "nlist": NLIST, "nprobe": npb, "alpha": alpha, "k": K,
-            "batch": BATCH, "n_train": n_train,
+            "batch": BATCH, "queries_per_timed_batch": roof["queries_per_batch"],
+            "n_train": n_train,
             "recall_at_10": round(rec10, 4), "recall_at_100": round(rec100, 4),
             "streaming": {"insert_batches": nbatches, "insert_vectors_per_s":
                           round(NINS / max(t_ins, 1e-9), 1),
@@ -992,28 +1009,27 @@ def trace_mode(torch, dev, ix, q, k, batch, nprobe, alpha, nsteps):
         torch.cuda.synchronize()
         ms.append(ev0.elapsed_time(ev1))
     print(json.dumps({"trace_steps": nsteps, "nprobe": nprobe, "alpha": alpha, "nq": nq,
-                      "batches_per_step": (nq + batch - 1) // batch,
+                      "batches_per_step": -(-nq // ix.call_plan(nq, k)["rows"]),
                       "scan_kernel": ix.scan_plan(k)[0],
                       "ms_per_step_hip_events": [round(x, 4) for x in ms]}), flush=True)
 
 
 def profile_mode(torch, dev, ix, q, k, batch, nprobe, alpha, nbatches):
     """A short, fixed workload for rocprofv3 counter runs: `nbatches` search
-    batches over distinct queries, then one elementwise float32 kernel that
+    batches of the size that a call over all of q runs, over distinct queries (the
+    first `nbatches` launches of each search kernel), then one elementwise float32 kernel that
     reads and writes 256 MiB; its FETCH_SIZE / WRITE_SIZE readings calibrate
     the counters."""
     ix.set_nprobe(nprobe)
     ix.set_alpha(alpha)
+    nq = q.shape[0]
+    batch = ix.call_plan(nq, k)["rows"]
     out_d = torch.empty((batch, k), dtype=torch.float32, device=dev)
     out_i = torch.empty((batch, k), dtype=torch.int32, device=dev)
-    nq = q.shape[0]
-    ix.set_timing(True)
     for s in range(nbatches):
         q0 = (s * batch) % max(1, nq - batch + 1)
         ix.search_device(q[q0:q0 + batch], k, out_d, out_i)
     torch.cuda.synchronize()
-    tm, nb = ix.timing()
-    ix.set_timing(False)
     # calibration: an elementwise float32 kernel that reads and writes 256 MiB
     src = torch.ones(64 << 20, dtype=torch.float32, device=dev)
     dst = torch.empty_like(src)
@@ -1028,9 +1044,8 @@ def profile_mode(torch, dev, ix, q, k, batch, nprobe, alpha, nbatches):
     for qq in qs:
         dbg = ix.search_debug(qq.cpu().numpy(), k)
         tot += int(sizes[dbg["probes"]].sum()) * ix.params.M
-    print(json.dumps({"profile_batches": nbatches, "nprobe": nprobe, "alpha": alpha,
-                      "scan_bytes_per_launch": tot / nbatches,
-                      "step_us_per_batch": {k2: round(v * 1000.0 / nb, 2) for k2, v in tm.items()},
+    print(json.dumps({"profile_batches": nbatches, "queries_per_batch": batch, "nprobe": nprobe,
+                      "alpha": alpha, "scan_bytes_per_launch": tot / nbatches,
                       "calibration_kernel": "torch.mul(float32[64Mi], 1.0)",
                       "calibration_bytes_each_way": 256 << 20}), flush=True)
 
