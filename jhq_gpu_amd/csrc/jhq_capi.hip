@@ -914,7 +914,7 @@ int merged_rows(jhq_index* ix) {
     const int B = ix->batch_size, P = std::min(ix->nprobe, ix->nlist);
     const int rck = ix->RC * ix->Kr;
     // (the pre-scan's pair limit holds only where it may be chosen: 4 M x 128, M 16,
-    // 64 probes, 2048 queries, B 64: 3260 us in batches of 64, 2535 in merged ones)
+    // 64 probes, 2048 queries, B 64: 3260 us in batches of 64, 2204 in merged ones)
     const bool prescan = ix->scan_kind == 2 || (ix->scan_kind == 0 && ix->M >= kMfmaMinM);
     struct Path {
         bool mfma;
@@ -926,7 +926,8 @@ int merged_rows(jhq_index* ix) {
     };
     auto path = [&](int k, int rows, Path* p) {
         const int ck = ceil_ck(ix->alpha, k);
-        p->mfma = prescan && jhq::mfma_scan_ok(ix->M, ix->d, ix->Ds, ix->K1D, ix->bpd, rows, P, ck, rck);
+        p->mfma = prescan && jhq::mfma_scan_ok(ix->M, ix->d, ix->Ds, ix->K1D, ix->bpd, rows, P, ck,
+                                               rck);
         p->sh = jhq::ScanShape{};
         return jhq::scan_plan(ix->M, ix->d, P, ck, ix->K1D, rows, ix->num_cu, &p->sh,
                               skew_eligible(ix), false, rck);
